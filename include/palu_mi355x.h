@@ -21,7 +21,7 @@
 extern "C" {
 #endif
 
-#define PALU_ABI_VERSION 14
+#define PALU_ABI_VERSION 15
 
 #define PALU_OK 0
 #define PALU_EINVAL 1       /* arguments outside the op's envelope */
@@ -357,6 +357,34 @@ int palu_linear_qkv(const void* x, long long ldx, int x_tiled, int rows, const v
                     void* q_out, void* k_cache, int k_layout, int k_col_offset, int k_group_stride, int k_width,
                     int k_rope, void* v_cache, int v_layout, int v_col_offset, int v_group_stride, int v_width,
                     int n_groups, int seq_len, palu_stream_t stream);
+
+/* ---- Prefill ----------------------------------------------------------------------------------------
+ * The attention of a prefill (the reference's palu_tt/attention.py:380-480 runs it as separate ttnn ops). */
+
+/* Latents of whole prompts into a cache: cache[u][g][p][0 .. width - 1] = src[(u * n_pos + p) * src_row_stride + g *
+ * src_group_stride ..] for u < users, p < n_pos (element strides, multiples of 8). cache is the first row's stream of
+ * group 0, its rows and groups batch_stride / group_stride elements apart, in any cache_layout (PALU_LAYOUT_ROWS,
+ * _TILED or _TILED_V; seq_len the positions of a stream, a multiple of 32 when tiled). Positions past n_pos keep what
+ * they hold. With cos_table / sin_table (fp32 [table_rows >= n_pos, 128], width 128, not _TILED_V) the rows are
+ * rotated at their positions first (the stock K path's heads). */
+int palu_latent_fill(void* cache, long long batch_stride, long long group_stride, const void* src,
+                     long long src_row_stride, long long src_group_stride, int users, int n_groups, int n_pos, int seq_len,
+                     int width, int cache_layout, const float* cos_table, const float* sin_table, int table_rows,
+                     palu_stream_t stream);
+
+/* Causal attention of `users` prompts of seq positions each, straight from the QKV projection's bf16 rows
+ * [users * seq][ld]: query heads at columns 0 .. n_heads * 128 - 1, group g's K latent at k_col_offset + g * r_k and V
+ * latent at v_col_offset + g * r_v. out[u * seq + p][h * 128 ..] (bf16, rows ld_out apart) = softmax(q K^T scale) V over
+ * positions 0 .. p with K = RoPE(lat u_k), V = lat u_v (u_k / u_v [n_kv][r][128]; NULL with one 128-wide group per KV
+ * head: the columns are K / V themselves). Keys, values, scores, probabilities and sums have fp32 precision; the
+ * result is rounded to bf16 once. Ranks are multiples of 16. workspace: palu_prefill_workspace_bytes, 16-byte aligned. */
+int palu_prefill_attention(const void* qkv, long long ld, int users, int seq, int n_heads, int n_kv, int n_groups,
+                           int k_col_offset, int r_k, const void* u_k, int v_col_offset, int r_v, const void* u_v,
+                           const float* cos_table, const float* sin_table, int table_rows, float scale, void* out,
+                           long long ld_out, void* workspace, size_t workspace_bytes, palu_stream_t stream);
+
+/* Workspace bytes of palu_prefill_attention (0 for invalid shapes): the rebuilt keys and values as operand tiles. */
+size_t palu_prefill_workspace_bytes(int users, int seq, int n_heads, int n_kv, int n_groups, int r_k, int r_v);
 
 #ifdef __cplusplus
 }

@@ -299,10 +299,32 @@ class PaluAttention(torch.nn.Module):
         x3 = x.reshape(-1, shape[-2], self.hidden_size).to(torch.bfloat16)          # [U, S, dim]
         U, S = x3.shape[0], x3.shape[1]
         assert 0 < S <= self.max_seq_len and user_id + U <= self.max_batch_size
+        if (U > 0 and user_id >= 0 and self.head_dim == 128 and decoder_ops.kernels_can_take(
+                x, self.wqkv.weight, self.wo, self.u_k, self.u_v, *(self._store(c) for c in self.layer_past))):
+            return self._prefill_kernels(x3.reshape(U * S, -1), U, user_id).reshape(*shape[:-1], self.hidden_size)
         outs = []
         for u in range(U):
             outs.append(self._prefill_one(x3[u], user_id + u))
         return torch.stack(outs).reshape(*shape[:-1], self.hidden_size)
+
+    @staticmethod
+    def _store(cache):
+        return cache if isinstance(cache, torch.Tensor) else cache.data
+
+    def _prefill_kernels(self, x2, U, user):
+        """The prompts of cache rows user .. user + U - 1 at once (x2 [U * S, dim]): one QKV projection, the latents (or
+        rotated K heads) into the caches, the prefill attention kernel and the output projection."""
+        xqkv = F.linear(x2, self.wqkv.plain())                              # [U S, nh hd + G (kw + r_v)]
+        keys, values = self.layer_past
+        n_pos, kw, G = x2.shape[0] // U, self.k_width, self.n_groups
+        k0 = self.n_heads * self.head_dim
+        v0 = k0 + G * kw
+        rot = (None, None) if self.recon_k else (self.cos, self.sin)
+        decoder_ops.fill_from(keys, user, xqkv, U, n_pos, k0, kw, *rot)
+        decoder_ops.fill_from(values, user, xqkv, U, n_pos, v0, self.r_v)
+        attn = decoder_ops.prefill_attention(xqkv, U, self.n_heads, self.n_kv_heads, G, k0, kw, self.u_k, v0, self.r_v,
+                                             self.u_v, self.cos, self.sin, self.scale)
+        return F.linear(attn, self.wo)
 
     def _prefill_one(self, x2, user):
         S = x2.shape[0]

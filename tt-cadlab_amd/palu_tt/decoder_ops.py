@@ -143,6 +143,89 @@ def append_from(cache, src: torch.Tensor, group_stride: int, width: int, pos: to
         _native.stream_handle(src.device)))
 
 
+def fill_from(cache, user: int, src: torch.Tensor, users: int, n_pos: int, col: int, width: int,
+              cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None) -> None:
+    """Whole prompts into a cache: cache[user + u, g, p, :] = src[u * n_pos + p, col + g * width : + width] for a
+    row-strided src [users * n_pos, ...] (the QKV projection's rows), positions past n_pos untouched. cache: LatentCache,
+    a row-major [B, G, S, width] bf16 tensor or a GroupedLatentCache (each group its first ranks[g] columns). With cos /
+    sin (fp32 [>= n_pos, 128]) the 128-wide rows are rotated at their positions first."""
+    _check(src, "src")
+    if src.dim() != 2 or src.stride(1) != 1 or src.shape[0] != users * n_pos:
+        raise RuntimeError(f"src must be a row-strided [{users * n_pos}, columns] view")
+    B, G, S, w = cache.shape
+    if not (0 <= user and user + users <= B and 0 < n_pos <= S) or w > width or src.shape[1] < col + G * width:
+        raise RuntimeError(f"{users} prompts of {n_pos} positions, {G} x {width} columns from {col}, do not fit")
+    store = cache.data if isinstance(cache, (LatentCache, GroupedLatentCache)) else cache
+    _check(store, "cache")
+    if not store.is_contiguous() or store.device != src.device:
+        raise RuntimeError("the cache must be contiguous and on the device of src")
+    layout = _native.LAYOUT_ROWS
+    if store is not cache:
+        layout = _native.LAYOUT_TILED if cache.role == "k" else _native.LAYOUT_TILED_V
+    if isinstance(cache, GroupedLatentCache):
+        row = S * sum(cache.ranks)
+        parts = [(user * row + S * sum(cache.ranks[:g]), row, 0, col + g * width, 1, r) for g, r in enumerate(cache.ranks)]
+    else:
+        if w != width:
+            raise RuntimeError(f"cache width {w} != fill width {width}")
+        parts = [(user * G * S * w, G * S * w, S * w, col, G, w)]
+    lib, stream = _native.load(), _native.stream_handle(src.device)
+    for off, sb, sg, c, groups, r in parts:
+        _native.check(lib.palu_latent_fill(
+            store.data_ptr() + 2 * off, sb, sg, src.data_ptr() + 2 * c, src.stride(0), width, users, groups, n_pos, S, r,
+            layout, _native.ptr(cos), _native.ptr(sin), 0 if cos is None else cos.shape[0], stream))
+
+
+def prefill_attention(qkv: torch.Tensor, users: int, n_heads: int, n_kv: int, n_groups: int, k_col: int, r_k: int,
+                      u_k: Optional[torch.Tensor], v_col: int, r_v: int, u_v: Optional[torch.Tensor], cos: torch.Tensor,
+                      sin: torch.Tensor, scale: float) -> torch.Tensor:
+    """Causal attention of `users` prompts from their QKV projection rows qkv [users * seq, ...] (bf16): query heads,
+    then group g's K latent at column k_col + g * r_k and V latent at v_col + g * r_v; K = RoPE(lat @ u_k), V = lat @ u_v
+    (None: the columns are K / V heads themselves), in fp32 precision throughout. Returns bf16 [users * seq, n_heads *
+    128]."""
+    _check(qkv, "qkv")
+    _check(cos, "cos", torch.float32)
+    _check(sin, "sin", torch.float32)
+    for t, n, r in ((u_k, "u_k", r_k), (u_v, "u_v", r_v)):
+        if t is not None:
+            _check(t, n)
+            if t.shape != (n_kv, r, 128) or not t.is_contiguous():
+                raise RuntimeError(f"{n} must be a contiguous [{n_kv}, {r}, 128] tensor")
+    rows = qkv.shape[0]
+    if qkv.dim() != 2 or qkv.stride(1) != 1 or users < 1 or rows % users or not (cos.is_contiguous() and sin.is_contiguous()):
+        raise RuntimeError("qkv must be a row-strided [users * seq, columns] view; cos and sin contiguous")
+    if qkv.shape[1] < max(n_heads * 128, k_col + n_groups * r_k, v_col + n_groups * r_v):
+        raise RuntimeError(f"qkv rows of {qkv.shape[1]} columns do not hold the heads and latents")
+    lib = _native.load()
+    dims = (users, rows // users, n_heads, n_kv, n_groups)
+    need = lib.palu_prefill_workspace_bytes(*dims, r_k, r_v)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=qkv.device)
+    out = torch.empty(rows, n_heads * 128, dtype=torch.bfloat16, device=qkv.device)
+    _native.check(lib.palu_prefill_attention(
+        _native.ptr(qkv), qkv.stride(0), *dims, k_col, r_k, _native.ptr(u_k), v_col, r_v, _native.ptr(u_v),
+        _native.ptr(cos), _native.ptr(sin), min(cos.shape[0], sin.shape[0]), float(scale), _native.ptr(out), out.stride(0),
+        _native.ptr(ws), ws.numel(), _native.stream_handle(qkv.device)))
+    return out
+
+
+def kernels_can_take(x: torch.Tensor, *weights) -> bool:
+    """Whether a forward over x may run on the library's kernels, which see data pointers only: a plain GPU tensor that
+    nothing records, traces or transforms (autograd on x or a weight, forward-mode tangents, functorch, tracing,
+    compiling and tensor subclasses take the torch path)."""
+    if type(x) is not torch.Tensor or not x.is_cuda:
+        return False
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.is_functorch_wrapped_tensor(x):
+        return False
+    if torch._C._len_torch_dispatch_stack() or any(
+            not isinstance(m, torch.utils._device.DeviceContext) for m in torch.overrides._get_current_function_mode_stack()):
+        return False                   # a dispatch or function mode (other than a default device) watches the torch calls
+    tensors = [t for t in (x, *weights) if t is not None]
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return not any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors) \
+        if torch.autograd.forward_ad._current_level >= 0 else True
+
+
 def tile_weight(w: torch.Tensor, rtw: int) -> torch.Tensor:
     """The [n, k] nn.Linear weight in the decode projection's tiled order for workgroups of rtw row tiles
     (a new contiguous tensor of the same bytes). Tile (rt, kt) of 16 output columns x 32 inputs is 1 KB,
