@@ -279,6 +279,7 @@ int palu_rope_rows(const void* src, long long src_row_stride, void* dst, const i
 #define PALU_LINEAR_BF16 0          /* y: bf16 [rows, n], rows ldy apart */
 #define PALU_LINEAR_F32_PARTIALS 1  /* y: fp32 [ks, rows, n], the k slices' partial sums, not added up */
 #define PALU_LINEAR_SWIGLU_TILED 2  /* y: bf16 [64, n / 2] tiled activations, silu(gate) * up (ks = 1) */
+#define PALU_LINEAR_SWIGLU_ROWS 3   /* palu_linear_rows only. y: bf16 [rows, n / 2], silu(gate) * up */
 
 /* Decode-step projection: y[r][c] = sum_k x[r][k] w[c][k] for rows = 1..64 (bf16 in, fp32 accumulate),
  * with w [n, k] given tiled for groups of rtw row tiles (palu_tt.decoder_ops.tile_weight: 16 x 32 tiles
@@ -360,6 +361,17 @@ int palu_linear_qkv(const void* x, long long ldx, int x_tiled, int rows, const v
 
 /* ---- Prefill ----------------------------------------------------------------------------------------
  * The attention of a prefill (the reference's palu_tt/attention.py:380-480 runs it as separate ttnn ops). */
+
+/* Projection of many rows: y[r][c] = sum_k x[r][k] w[c][k] for any number of bf16 rows (ldx apart, a multiple of 8), over
+ * the weight as palu_linear_tiled takes it (tiled for groups of rtw row tiles), fp32 accumulate. y_mode PALU_LINEAR_BF16:
+ * y bf16 rows ldy apart; PALU_LINEAR_SWIGLU_ROWS: w holds gate and up rows interleaved eight at a time and y receives
+ * silu(gate) * up (bf16, n / 2 columns). ldy a multiple of 4. workspace: palu_linear_rows_workspace_bytes (fp32 sums of k
+ * slices), 16-byte aligned. */
+int palu_linear_rows(const void* x, long long ldx, int rows, const void* w_tiled, int n, int k, int rtw, void* y,
+                     long long ldy, int y_mode, void* workspace, size_t workspace_bytes, palu_stream_t stream);
+
+/* Workspace bytes of palu_linear_rows (0 when the product is not split). */
+size_t palu_linear_rows_workspace_bytes(int rows, int n, int k, int y_mode);
 
 /* Latents of whole prompts into a cache: cache[u][g][p][0 .. width - 1] = src[(u * n_pos + p) * src_row_stride + g *
  * src_group_stride ..] for u < users, p < n_pos (element strides, multiples of 8). cache is the first row's stream of

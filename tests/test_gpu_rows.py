@@ -1,0 +1,52 @@
+"""The prefill projection kernel (palu_linear_rows) against 64-bit torch.
+
+Bound: half a bf16 step at the result plus the fp32 sum's rounding. A dot product of k terms is k / 32 MFMAs accumulated
+one after another (and up to 16 slices added), each addition rounding by at most 2^-24 of the running sum, which the sum
+of the terms' magnitudes bounds."""
+import pytest
+import torch
+
+from palu_tt import decoder_ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _half_step(e):
+    return torch.ldexp(torch.ones_like(e), torch.frexp(e).exponent - 9)
+
+
+def _case(m, n, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(m, k + 8, generator=g).to(torch.bfloat16).cuda()[:, :k]
+    w = (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    return x, w
+
+
+# rows around the 128-row blocks; columns that are no whole workgroup, and last groups of fewer row tiles; k of one
+# tile, an odd number of tiles, every remainder of the four-stage round, and lengths that split (odd slices among them)
+@pytest.mark.parametrize("m,n,k,rtw", [
+    (65, 16, 32, 1), (127, 48, 64, 2), (128, 80, 96, 3), (129, 272, 160, 4), (300, 1040, 224, 7), (70, 528, 288, 8),
+    (200, 512, 352, 5), (257, 64, 416, 6), (1, 96, 512, 2), (100, 128, 2080, 1), (66, 256, 4128, 3), (500, 2064, 1056, 7),
+    (1030, 4112, 128, 2)])
+def test_linear_rows(gpu, m, n, k, rtw):
+    x, w = _case(m, n, k, m + n + k)
+    y = ops.linear_rows(x, ops.tile_weight(w, rtw), rtw).double()
+    exp = x.double() @ w.double().T
+    mag = x.double().abs() @ w.double().abs().T
+    bound = _half_step(exp) * 1.001 + (k / 32 + 24) * 2.0 ** -24 * mag
+    assert ((y - exp).abs() / bound).max().item() <= 1.0
+
+
+@pytest.mark.parametrize("m,f,k,rtw", [(65, 32, 32, 1), (130, 96, 224, 7), (257, 544, 96, 3), (128, 1024, 512, 4), (33, 64, 64, 8)])
+def test_linear_rows_swiglu(gpu, m, f, k, rtw):
+    x, g = _case(m, f, k, f + k)
+    u = _case(1, f, k, f + k + 1)[1]
+    y = ops.linear_rows(x, ops.tile_weight(ops.interleave_gate_up(g, u), rtw), rtw, swiglu=True).double()
+    xd, gd, ud = x.double(), g.double(), u.double()
+    gv, uv = xd @ gd.T, xd @ ud.T
+    exp = torch.nn.functional.silu(gv) * uv
+    # the fp32 sums of gate and up (|d silu| <= 1.1), and the fp32 exponential and division: a few 2^-22 of the result
+    eps = (k / 32 + 24) * 2.0 ** -24
+    bound = _half_step(exp) * 1.001 + 1.1 * eps * (xd.abs() @ gd.abs().T) * uv.abs() + eps * gv.abs() * (xd.abs() @ ud.abs().T) \
+        + 2.0 ** -20 * exp.abs()
+    assert ((y - exp).abs() / bound).max().item() <= 1.0

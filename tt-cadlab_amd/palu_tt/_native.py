@@ -54,6 +54,8 @@ _SIGNATURES = {
     "palu_linear_residual": (_i, [_vp, _ll, _i, _i, _vp, _i, _i, _i, _vp, _ll, _vp, _vp]),
     "palu_linear_qkv": (_i, [_vp, _ll, _i, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _i, _i, _i, _i, _i,
                              _vp, _i, _i, _i, _i, _i, _i, _vp]),
+    "palu_linear_rows": (_i, [_vp, _ll, _i, _vp, _i, _i, _i, _vp, _ll, _i, _vp, _sz, _vp]),
+    "palu_linear_rows_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "palu_latent_fill": (_i, [_vp, _ll, _ll, _vp, _ll, _ll, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _vp]),
     "palu_prefill_attention": (_i, [_vp, _ll, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _f, _vp, _ll,
                                     _vp, _sz, _vp]),

@@ -301,7 +301,7 @@ class PaluAttention(torch.nn.Module):
         assert 0 < S <= self.max_seq_len and user_id + U <= self.max_batch_size
         if (U > 0 and user_id >= 0 and self.head_dim == 128 and decoder_ops.kernels_can_take(
                 x, self.wqkv.weight, self.wo, self.u_k, self.u_v, *(self._store(c) for c in self.layer_past))):
-            return self._prefill_kernels(x3.reshape(U * S, -1), U, user_id).reshape(*shape[:-1], self.hidden_size)
+            return self._prefill_kernels(x3.reshape(U * S, -1).contiguous(), U, user_id).reshape(*shape[:-1], self.hidden_size)
         outs = []
         for u in range(U):
             outs.append(self._prefill_one(x3[u], user_id + u))
@@ -314,7 +314,7 @@ class PaluAttention(torch.nn.Module):
     def _prefill_kernels(self, x2, U, user):
         """The prompts of cache rows user .. user + U - 1 at once (x2 [U * S, dim]): one QKV projection, the latents (or
         rotated K heads) into the caches, the prefill attention kernel and the output projection."""
-        xqkv = F.linear(x2, self.wqkv.plain())                              # [U S, nh hd + G (kw + r_v)]
+        xqkv = self.wqkv.rows(x2)                                           # [U S, nh hd + G (kw + r_v)]
         keys, values = self.layer_past
         n_pos, kw, G = x2.shape[0] // U, self.k_width, self.n_groups
         k0 = self.n_heads * self.head_dim

@@ -433,6 +433,20 @@ def linear_qkv(x: torch.Tensor, w_tiled: torch.Tensor, rtw: int, pos: torch.Tens
     return q_out
 
 
+def linear_rows(x: torch.Tensor, w_tiled: torch.Tensor, rtw: int, swiglu: bool = False) -> torch.Tensor:
+    """x @ w.T for any number of rows (a prefill's) with w given by tile_weight(w, rtw) ([n, k]): bf16 [rows, n], or with
+    swiglu (w_tiled tiled from interleave_gate_up) silu(gate) * up, [rows, n / 2]. x: a row-strided [rows, k] view."""
+    rows, n, k = _operands(x, w_tiled, False, None)
+    lib = _native.load()
+    mode = 3 if swiglu else 0
+    need = lib.palu_linear_rows_workspace_bytes(rows, n, k, mode)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    out = torch.empty(rows, n // 2 if swiglu else n, dtype=torch.bfloat16, device=x.device)
+    _native.check(lib.palu_linear_rows(_native.ptr(x), x.stride(0), rows, _native.ptr(w_tiled), n, k, rtw, _native.ptr(out),
+                                       out.stride(0), mode, _native.ptr(ws), need, _native.stream_handle(x.device)))
+    return out
+
+
 def interleave_gate_up(w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
     """[2 ffn, k] with gate and up rows interleaved eight at a time (rows 16 j .. 16 j + 7: gate rows
     8 j .. 8 j + 7, then the up rows of the same outputs), the weight linear_tiled's "swiglu" mode takes."""
@@ -615,6 +629,15 @@ class DecodeLinear:
         return linear_qkv(x, self.weight, self.rtw, pos, cos, sin, n_heads, keys, k_col_offset, k_group_stride,
                           k_width, values, v_col_offset, v_group_stride, v_width, k_rope=k_rope, x_tiled=x_tiled,
                           rows=rows)
+
+    def rows(self, x: torch.Tensor) -> torch.Tensor:
+        """The projection of a prefill's rows [rows, k] (any number) as bf16 rows: x @ w.T, or silu(gate) * up of a pair.
+        A tiled weight is multiplied as it is held, up to 64 rows by the decode step's kernel."""
+        if not self.tiled:
+            return self(x)
+        if not self.gate_up and x.shape[0] <= 64:
+            return self(x)
+        return linear_rows(x, self.weight, self.rtw, swiglu=self.gate_up)
 
     def plain(self) -> torch.Tensor:
         if not self.tiled:

@@ -116,10 +116,28 @@ class Transformer(torch.nn.Module):
         logits of the last position of every row, [U, vocab]."""
         eps = self.args.norm_eps
         h = self.tok_embeddings[tokens]                                  # [U, S, dim]
+        if tokens.numel() > 0 and self.args.dim % 8 == 0 and self.args.dim <= 8192 and decoder_ops.kernels_can_take(h):
+            return self._prefill_kernels(h, user_id)
         for L in self.layers:
             h = h + L["attn"].forward_prefill(rms_norm(h, L["attn_norm"], eps), user_id=user_id)
             h = h + self._ffn(L, rms_norm(h, L["ffn_norm"], eps))
         return F.linear(rms_norm(h[:, -1], self.norm_w, eps), self.output.plain()).float()
+
+    def _prefill_kernels(self, h, user_id):
+        """prefill() of the embedded prompts h [U, S, dim] on the library's kernels: RMSNorm with the residual add, the
+        projections over the weights as they are held, SwiGLU in the gate / up epilogue; only the last position goes
+        through the head."""
+        U, S, dim = h.shape
+        eps = self.args.norm_eps
+        h, f = h.view(U * S, dim), None
+        for L in self.layers:
+            y = decoder_ops.rmsnorm(h, L["attn_norm"], eps, res=f, h_out=None if f is None else h)
+            o = L["attn"].forward_prefill(y.view(U, S, dim), user_id=user_id).view(U * S, dim)
+            y = decoder_ops.rmsnorm(h, L["ffn_norm"], eps, res=o, h_out=h)
+            f = L["w2"].rows(L["w13"].rows(y))
+        last = lambda t: t.view(U, S, dim)[:, -1].contiguous()
+        y = decoder_ops.rmsnorm(last(h), self.norm_w, eps, res=last(f))
+        return self.output.rows(y).float()
 
     @torch.no_grad()
     def decode(self, tokens: torch.Tensor, current_pos: torch.Tensor, greedy: bool = False) -> torch.Tensor:
