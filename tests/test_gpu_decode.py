@@ -449,3 +449,32 @@ def test_row_major_v_width_in_16s_is_refused(gpu):
     q, k_lat, u_k, v, pos, cos, sin = _inputs(2, 256, 64, 48)
     with pytest.raises(RuntimeError, match="r_v must be a multiple of 32"):
         _run_fused(gpu, q, k_lat, u_k, v, pos, cos, sin, 256)
+
+
+@pytest.mark.parametrize("B,nkv,S", [(1, 1, 65536), (1, 8, 4096), (3, 2, 8192), (2, 8, 512), (33, 8, 600)])
+def test_split_items_merge_on_every_replay(gpu, B, nkv, S):
+    """Items cut into 1 to 256 chunks, whose done flags a replayed launch meets again with the same tag: every
+    replay, at other positions and with eager calls and fresh memory in between, equals the unreplayed call."""
+    g = torch.Generator().manual_seed(S + B)
+    lat = lambda: torch.randn(B, nkv, S, 32, generator=g).to(gpu, torch.bfloat16)
+    k, v, q = lat(), lat(), torch.randn(1, B, 4 * nkv, HD, generator=g).to(gpu, torch.bfloat16)
+    u_k = (torch.randn(nkv, 32, HD, generator=g) / 32 ** 0.5).to(torch.bfloat16)
+    w = ref.w_rot_from_u_k(u_k.float())[None].to(gpu, torch.bfloat16)
+    cos, sin = ref.cos_sin_tables(HD, S, THETA, LLAMA3)
+    cs = ref.cs_table(cos, sin, S)[None, None].to(gpu)
+    pos = torch.full((B,), S - 1, dtype=torch.int32, device=gpu)
+    call = lambda: fused.palu_sdpa_decode(q, k, w, cs, v, 32, pos, scale=HD ** -0.5, out_dtype=torch.float32, deterministic=True)
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for i in range(5):
+        pos.copy_(torch.randint(0, S, (B,), generator=g).to(torch.int32) if i else pos)
+        torch.empty(1 << 20, device=gpu).fill_(i)
+        graph.replay()
+        got = out.clone()
+        assert torch.equal(got, call()), f"replay {i}"
+    pos_h = pos.cpu().long()
+    exp = ref.reference_decode(q.float().cpu(), k.float().cpu(), u_k.float(), v.float().cpu(), pos_h, cos, sin, HD ** -0.5)
+    _check(got.cpu(), exp)

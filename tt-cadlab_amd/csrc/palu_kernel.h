@@ -85,7 +85,7 @@ struct DecodeArgs {
   int n_splits;
   int n_wg;               // M-LRD / stock decode: workgroups launched; n_wg > B * n_kv splits items by length
   int balanced;           // 1 when n_wg > B * n_kv (length-aware chunks, merged through ws)
-  unsigned long long epoch;  // balanced: this call's tag for the items' chunk counters (CHUNK_TAG | call number)
+  unsigned long long epoch;  // balanced: this call's value of a chunk's done flag (CHUNK_TAG | call number)
   int deterministic;      // 1: wave w takes blocks w, w + NW, ... (reproducible); 0: blocks from a counter
   int out_tiled;          // 1: out in the 64-row tiled activation layout of the next projection (B <= 64)
   int grouped_streams;    // grouped latents stored compactly, each group at its own ranks (PALU_LAYOUT_TILED_GROUPED)
@@ -118,8 +118,8 @@ struct DecodeArgs {
 int fail(int code, const char* fmt, ...);
 extern thread_local char g_err[1024];
 
-// Last-finisher counters (count_done; the chunks of split decode items): bits 63..48 a fixed tag,
-// 47..16 the call number (next_epoch, one per launch that counts), 15..0 the count so far.
+// Value of the done flags of split decode items: bits 63..48 a fixed tag, 47..16 the call number (next_epoch,
+// one per launch with split items), 15..0 zero.
 constexpr unsigned long long CHUNK_TAG = 0xA5C3ull << 48;
 unsigned long long next_epoch();   // defined in palu_capi.hip
 
@@ -184,8 +184,8 @@ inline size_t ws_bytes(int items, int n_splits, int rv) {
 inline int decode_workgroups(int items) { return ((items + TARGET_WGS - 1) / TARGET_WGS) * TARGET_WGS; }
 inline size_t decode_ws_bytes(int items, int rv) {
   const int wg = decode_workgroups(items);
-  // partial slots [wg][16][rv + 2] floats, then one 8-byte chunk counter per item
-  return wg == items ? 0 : (size_t)wg * 16 * (rv + 2) * sizeof(float) + (size_t)items * sizeof(unsigned long long);
+  // partial slots [wg][16][rv + 2] floats, then one 8-byte done flag per workgroup
+  return wg == items ? 0 : (size_t)wg * 16 * (rv + 2) * sizeof(float) + (size_t)wg * sizeof(unsigned long long);
 }
 
 
@@ -359,8 +359,8 @@ __device__ __forceinline__ float wave_sum_xor48(float x) {
 // ---- length-aware chunk plan ------------------------------------------------------------------
 // With `items` = B * n_kv work items and G = n_wg > items workgroups, every workgroup derives the same
 // plan from cur_pos: chunks are whole pairs of blocks (64 positions); row b has np_b pairs; the chunk
-// length T (pairs) is the smallest of 64 candidates between ceil(W / G) and ceil(W / (G - items))
-// (W = n_kv * sum_b np_b) for which n_kv * sum_b max(1, ceil(np_b / T)) <= G. The upper end always
+// length T (pairs) is the smallest of 64 candidates from lo = max(ceil(W / G), the least chunk) up to
+// max(lo, ceil(W / (G - items))) (W = n_kv * sum_b np_b) for which n_kv * sum_b max(1, ceil(np_b / T)) <= G. The upper end always
 // qualifies, since sum_b max(1, ceil(np_b / T)) <= W / (n_kv T) + B. Item (b, kvh) is cut into
 // n_b = max(1, ceil(np_b / T)) near-equal chunks; chunks are numbered row by row, then KV head by KV
 // head, and chunk number = workgroup index = workspace slot.
@@ -398,10 +398,17 @@ __device__ __forceinline__ int row_pairs(const DecodeArgs& a, int b) { return (r
 __device__ int plan_chunk_pairs(const DecodeArgs& a) {
   const int lane = threadIdx.x & 63;
   const int G = a.n_wg, items = a.B * a.n_kv;
-  int W = 0;
-  for (int b = 0; b < a.B; ++b) W += row_pairs(a, b);
+  int W = 0, longest = 0;
+  for (int b = 0; b < a.B; ++b) {
+    const int np = row_pairs(a, b);
+    W += np;
+    longest = max(longest, np);
+  }
   W *= a.n_kv;
-  const int lo = max(1, (W + G - 1) / G);
+  // A chunk costs a merge, and its waves work side by side: no chunk is shorter than 4 pairs, and items of up to 8 pairs
+  // (one per wave) stay whole. Measured with the least chunk 1 / 4 / 8 pairs: 1 x 1024 positions 11.4 / 10.9 / 11.8 us,
+  // 1 x 4096 14.3 / 12.6 / 12.9, 4 x 2000 13.5 / 13.1 / 13.9, 1 x 128 10.7 / 8.5 / 8.5, 12 x 500 16.2 / 15.8 / 14.6.
+  const int lo = max(longest <= 8 ? 8 : 4, (W + G - 1) / G);
   const int hi = max(lo, (W + (G - items) - 1) / (G - items));
   const int step = max(1, (hi - lo + 62) / 63);
   const int T = lo + lane * step;           // lane 63: T >= hi
@@ -457,46 +464,44 @@ __device__ __forceinline__ float4 load4f<__bf16>(const __bf16* p) {
   return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
 }
 
-// Last-finisher counting across the workgroups of one launch. Each of nc workgroups that produce parts
-// of one result has written its part with system-scope stores (global stores that write through past
-// the XCD's L2 to memory) and waited for them to complete; then one thread calls count_done, which adds
-// the workgroup to the result's 8-byte counter with a system-scope compare-and-swap and returns true for
-// the workgroup whose count completes the result. That workgroup reads the parts with system-scope loads
-// (from memory, whichever XCD wrote them: no L2 write-back or invalidate, no fence) and leaves the
-// counter at zero. A counter word carries a fixed tag and the call number in its upper 48 bits (tag,
-// from next_epoch; its low 16 bits zero) and the count below; a word with other upper bits (another
-// call's, memory never written) counts as zero, so counters need no clearing between calls.
-__device__ __forceinline__ bool count_done(unsigned long long* ctr, unsigned long long tag, int nc) {
-  unsigned long long old = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM), nw;
-  int done;
-  do {
-    done = (((old & ~0xFFFFull) == tag) ? (int)(old & 0xFFFF) : 0) + 1;
-    nw = tag | (unsigned long long)(done == nc ? 0 : done);
-  } while (!__hip_atomic_compare_exchange_strong(ctr, &old, nw, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_SYSTEM));
-  return done == nc;
-}
-
-// The workgroup-wide step before and around count_done: every thread's system-scope stores complete,
-// thread 0 counts, and the answer (uniform) comes back through the LDS word *flag.
-__device__ __forceinline__ bool workgroup_count_done(unsigned long long* ctr, unsigned long long tag, int nc, int* flag) {
+// The chunks of a split item: chunk `mine` of nc has written its part with system-scope stores, which write
+// through past the XCD's L2 to memory (system-scope loads read from there, whichever XCD wrote: no L2
+// write-back or invalidate, no fence). Its done flag, one word per chunk, is set to this call's tag once
+// those stores have completed, and then all the item's flags are read: true (uniform) where every one is
+// set. Each chunk sets its flag before it reads the others', so the chunk whose flag lands last sees them all;
+// another may see them all as well, and both then write the same result. Whoever does clears the flags
+// (every chunk has set its own by then), so that a replayed launch, whose tag is the same, starts from
+// cleared ones; any other word (another call's tag, memory never written) is not set. A flag costs one store and
+// one parallel read, however many chunks there are: a counter shared by an item's chunks took a
+// compare-and-swap each, one after the other (one row of 1024 positions, 8 items of 16 chunks: 24.1 us
+// a call against 11.4; one row of 8192: 51.5 against 14.4).
+__device__ __forceinline__ bool chunks_all_done(unsigned long long* flags, unsigned long long tag, int nc, int mine, int* flag) {
   __builtin_amdgcn_s_waitcnt(0);            // this thread's part stores have completed
   __syncthreads();
-  if (threadIdx.x == 0) flag[0] = count_done(ctr, tag, nc) ? 1 : 0;
+  if (threadIdx.x < 64) {
+    if (threadIdx.x == 0) __hip_atomic_store(flags + mine, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the flag is in memory before the others are read
+    bool set = true;
+    for (int i = threadIdx.x; i < nc; i += 64)
+      set = set && __hip_atomic_load(flags + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == tag;
+    const bool all = __all(set);
+    if (all)
+      for (int i = threadIdx.x; i < nc; i += 64)
+        __hip_atomic_store(flags + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) flag[0] = all ? 1 : 0;
+  }
   __syncthreads();
   return flag[0] != 0;
 }
 
 // A split item's chunks merge inside the decode launch (no second launch): each chunk's workgroup has
-// written its partial (O, m, l) with system-scope stores, counts itself into the item's counter, and the
-// workgroup that completes the item writes out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), chunks in
-// order: the result does not depend on which workgroup finishes last. smem: any LDS word no wave reads
-// any more.
+// written its partial (O, m, l) with system-scope stores, and the workgroup that finds the item complete
+// writes out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), chunks in order: the result does not depend
+// on which workgroup that is. smem: any LDS word no wave reads any more.
 template <int RV, int NW, typename OutT>
 __device__ __forceinline__ void merge_split_item(const DecodeArgs& a, char* smem, int first, int nc, int b, int kvh) {
-  unsigned long long* ctr =
-      reinterpret_cast<unsigned long long*>(a.ws + (long long)a.n_wg * 16 * (RV + 2)) + (b * a.n_kv + kvh);
-  if (!workgroup_count_done(ctr, a.epoch, nc, reinterpret_cast<int*>(smem))) return;   // uniform
+  unsigned long long* flags = reinterpret_cast<unsigned long long*>(a.ws + (long long)a.n_wg * 16 * (RV + 2)) + first;
+  if (!chunks_all_done(flags, a.epoch, nc, (int)blockIdx.x - first, reinterpret_cast<int*>(smem))) return;   // uniform
   constexpr int MC = 8;                     // chunk partials loaded together per round trip
   constexpr long long SLOT = 16 * (RV + 2);
   for (int e = threadIdx.x; e < a.rep * RV; e += NW * 64) {
