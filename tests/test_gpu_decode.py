@@ -451,7 +451,7 @@ def test_row_major_v_width_in_16s_is_refused(gpu):
         _run_fused(gpu, q, k_lat, u_k, v, pos, cos, sin, 256)
 
 
-@pytest.mark.parametrize("B,nkv,S", [(1, 1, 65536), (1, 8, 4096), (3, 2, 8192), (2, 8, 512), (33, 8, 600)])
+@pytest.mark.parametrize("B,nkv,S", [(1, 1, 65536), (1, 8, 4096), (3, 2, 8192), (2, 8, 512), (33, 8, 600), (65, 8, 300), (70, 1, 2000)])
 def test_split_items_merge_on_every_replay(gpu, B, nkv, S):
     """Items cut into 1 to 256 chunks, whose done flags a replayed launch meets again with the same tag: every
     replay, at other positions and with eager calls and fresh memory in between, equals the unreplayed call."""

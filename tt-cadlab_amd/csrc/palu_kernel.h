@@ -359,8 +359,8 @@ __device__ __forceinline__ float wave_sum_xor48(float x) {
 // ---- length-aware chunk plan ------------------------------------------------------------------
 // With `items` = B * n_kv work items and G = n_wg > items workgroups, every workgroup derives the same
 // plan from cur_pos: chunks are whole pairs of blocks (64 positions); row b has np_b pairs; the chunk
-// length T (pairs) is the smallest of 64 candidates from lo = max(ceil(W / G), the least chunk) up to
-// max(lo, ceil(W / (G - items))) (W = n_kv * sum_b np_b) for which n_kv * sum_b max(1, ceil(np_b / T)) <= G. The upper end always
+// length T (pairs) is the smallest from lo = max(ceil(W / G), the least chunk) up to max(lo, ceil(W / (G - items)))
+// (W = n_kv * sum_b np_b) for which n_kv * sum_b max(1, ceil(np_b / T)) <= G. The upper end always
 // qualifies, since sum_b max(1, ceil(np_b / T)) <= W / (n_kv T) + B. Item (b, kvh) is cut into
 // n_b = max(1, ceil(np_b / T)) near-equal chunks; chunks are numbered row by row, then KV head by KV
 // head, and chunk number = workgroup index = workspace slot.
@@ -390,33 +390,79 @@ __device__ __forceinline__ int clamp_len(const DecodeArgs& a, int pos) {
 }
 __device__ __forceinline__ int row_len(const DecodeArgs& a, int b) { return clamp_len(a, load_uniform(a.cur_pos, b)); }
 
-__device__ __forceinline__ int row_pairs(const DecodeArgs& a, int b) { return (row_len(a, b) + 63) >> 6; }
+// Inclusive prefix sum over the wave's lanes (six DPP adds, no LDS).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr 1, 2, 4, 8: within rows of 16 lanes
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast 15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ int wave_sum_i(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
 
-// The plan's chunk length T in pairs (the same value in every lane of every wave that calls it). The
-// rows' positions are read through the scalar cache: one line holds 16 rows, so B rows cost a miss per
-// 16 rows and hits for the rest.
-__device__ int plan_chunk_pairs(const DecodeArgs& a) {
+// The row length of row r0 + lane (0 past the batch).
+__device__ __forceinline__ int lane_row_len(const DecodeArgs& a, int r0) {
+  const int r = r0 + (int)(threadIdx.x & 63);
+  const int len = clamp_len(a, a.cur_pos[min(r, a.B - 1)]);
+  return r < a.B ? len : 0;
+}
+
+// A chunk of the plan: chunk j of the n chunks of row b's item of KV head kvh (b < 0: past the last chunk).
+struct Chunk {
+  int b, kvh, j, n, np, len;
+};
+
+// Workgroup gid's chunk (uniform). Every wave computes the whole plan, a lane to a row and 64 rows at a time;
+// len0 is lane_row_len of the first 64. Going through the rows one by one with scalar loads took
+// 1 us for every 5 to 10 rows (12 rows of 500 positions: 14.6 us a call against 11.2; 20 of 200: 14.2, 9.3; 48 of 2048:
+// 60.7, 43; 60 of up to 300: 46.6, 23.2, where every workgroup plans twice a CU).
+__device__ __forceinline__ Chunk plan_chunk(const DecodeArgs& a, int gid, int len0) {
   const int lane = threadIdx.x & 63;
   const int G = a.n_wg, items = a.B * a.n_kv;
+  auto pairs = [&](int r0) { return ((r0 == 0 ? len0 : lane_row_len(a, r0)) + 63) >> 6; };
   int W = 0, longest = 0;
-  for (int b = 0; b < a.B; ++b) {
-    const int np = row_pairs(a, b);
-    W += np;
-    longest = max(longest, np);
+  for (int r0 = 0; r0 < a.B; r0 += 64) {
+    const int np = pairs(r0);
+    W += wave_sum_i(np);
+    longest |= __any(np > 8) ? 1 : 0;
   }
   W *= a.n_kv;
   // A chunk costs a merge, and its waves work side by side: no chunk is shorter than 4 pairs, and items of up to 8 pairs
   // (one per wave) stay whole. Measured with the least chunk 1 / 4 / 8 pairs: 1 x 1024 positions 11.4 / 10.9 / 11.8 us,
   // 1 x 4096 14.3 / 12.6 / 12.9, 4 x 2000 13.5 / 13.1 / 13.9, 1 x 128 10.7 / 8.5 / 8.5, 12 x 500 16.2 / 15.8 / 14.6.
-  const int lo = max(longest <= 8 ? 8 : 4, (W + G - 1) / G);
-  const int hi = max(lo, (W + (G - items) - 1) / (G - items));
-  const int step = max(1, (hi - lo + 62) / 63);
-  const int T = lo + lane * step;           // lane 63: T >= hi
-  const FDiv fT = make_fdiv(T);
-  int C = 0;
-  for (int b = 0; b < a.B; ++b) C += max(1, ceil_fdiv(row_pairs(a, b), fT));
-  const unsigned long long ok = __ballot(C * a.n_kv <= G);
-  return lo + __builtin_ctzll(ok) * step;
+  int lo = max(longest ? 4 : 8, (W + G - 1) / G);
+  int hi = max(lo, (W + (G - items) - 1) / (G - items));
+  auto row_chunks = [&](int r0, FDiv fT) { return r0 + lane < a.B ? max(1, ceil_fdiv(pairs(r0), fT)) : 0; };
+  while (lo < hi) {                         // uniform
+    const int mid = (lo + hi) >> 1;
+    const FDiv fT = make_fdiv(mid);
+    int C = 0;
+    for (int r0 = 0; r0 < a.B; r0 += 64) C += wave_sum_i(row_chunks(r0, fT));
+    if (C * a.n_kv <= G) hi = mid;
+    else lo = mid + 1;
+  }
+  const FDiv fT = make_fdiv(hi);
+  int base = 0;
+  for (int r0 = 0; r0 < a.B; r0 += 64) {
+    const int c = row_chunks(r0, fT), incl = wave_scan(c * a.n_kv);
+    const unsigned long long past = __ballot(gid < base + incl);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      Chunk k;
+      k.b = r0 + l;
+      k.n = __builtin_amdgcn_readlane(c, l);
+      k.len = __builtin_amdgcn_readlane(r0 == 0 ? len0 : lane_row_len(a, r0), l);
+      k.np = (k.len + 63) >> 6;
+      const int at = gid - (base + __builtin_amdgcn_readlane(incl, l) - a.n_kv * k.n);
+      k.kvh = fdiv(at, make_fdiv(k.n));
+      k.j = at - k.kvh * k.n;
+      return k;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return Chunk{-1, 0, 0, 1, 0, 0};
 }
 
 // LDS map of one workgroup (latent mode; full-K mode keeps only the merge buffer and the counter):
@@ -576,6 +622,10 @@ void palu_decode_kernel(const DecodeArgs a) {
   const int n = lane & 15, g = lane >> 4;
   _Float16* qx = reinterpret_cast<_Float16*>(smem + SM::QX_OFFSET + w * SM::QX_WAVE_BYTES);
 
+  // The plan's first loads go ahead of everything else.
+  int len0 = 0;
+  if (a.balanced) len0 = lane_row_len(a, 0);
+
   // Latent mode: the angle-table rows are the same for every workgroup and depend on nothing below, so
   // their loads are issued first, ahead of the plan. Rows t < 64 serve the K rotation, 64*Lo (Lo < 16)
   // and 1024*H the query's pair base; one coalesced row per wave load.
@@ -612,23 +662,15 @@ void palu_decode_kernel(const DecodeArgs a) {
     kvh = item - b * a.n_kv;
     s_lo = 0;
   } else {
-    const FDiv fT = make_fdiv(plan_chunk_pairs(a));
-    int base = 0, rb = -1, np = 0;
-    const int gid = blockIdx.x;
-    for (int r = 0; r < a.B; ++r) {
-      np = row_pairs(a, r);
-      n_chunks = max(1, ceil_fdiv(np, fT));
-      if (gid < base + a.n_kv * n_chunks) { rb = r; break; }
-      base += a.n_kv * n_chunks;
-    }
-    if (rb < 0) return;                     // past the plan's last chunk (uniform: no barrier reached)
-    const FDiv fn = make_fdiv(n_chunks);
-    b = rb;
-    kvh = fdiv(gid - base, fn);
-    const int j = gid - base - kvh * n_chunks;
-    first_chunk = gid - j;                  // the item's chunks are workgroups first_chunk .. + n_chunks - 1
-    s_lo = 64 * fdiv(j * np, fn);
-    s_hi = min(row_len(a, b), 64 * fdiv((j + 1) * np, fn));
+    const Chunk ck = plan_chunk(a, blockIdx.x, len0);
+    if (ck.b < 0) return;                   // past the plan's last chunk (uniform: no barrier reached)
+    b = ck.b;
+    kvh = ck.kvh;
+    n_chunks = ck.n;
+    first_chunk = (int)blockIdx.x - ck.j;   // the item's chunks are workgroups first_chunk .. + n_chunks - 1
+    const FDiv fn = make_fdiv(ck.n);
+    s_lo = 64 * fdiv(ck.j * ck.np, fn);
+    s_hi = min(ck.len, 64 * fdiv((ck.j + 1) * ck.np, fn));
   }
   b = __builtin_amdgcn_readfirstlane(b);
   kvh = __builtin_amdgcn_readfirstlane(kvh);
