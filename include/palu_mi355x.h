@@ -21,7 +21,7 @@
 extern "C" {
 #endif
 
-#define PALU_ABI_VERSION 15
+#define PALU_ABI_VERSION 16
 
 #define PALU_OK 0
 #define PALU_EINVAL 1       /* arguments outside the op's envelope */
@@ -358,6 +358,21 @@ int palu_linear_qkv(const void* x, long long ldx, int x_tiled, int rows, const v
                     void* q_out, void* k_cache, int k_layout, int k_col_offset, int k_group_stride, int k_width,
                     int k_rope, void* v_cache, int v_layout, int v_col_offset, int v_group_stride, int v_width,
                     int n_groups, int seq_len, palu_stream_t stream);
+
+/* The decode step of per-head latents without the fused op (the reference's default, palu_tt/attention.py:657-710): the
+ * keys K[p] = RoPE_p(lat[p] u_k) of positions 0 .. min(cur_pos[b], recon_len - 1) are rebuilt into the workspace (bf16,
+ * rounded once) and the stock flash-decode runs over them and the V latent.
+ *   q [B, n_q, 128] bf16; k_latent [B, n_kv, seq_len, r_k], v_latent [B, n_kv, seq_len, r_v] bf16 in cache_layout
+ *   (PALU_LAYOUT_ROWS or _TILED); u_k [n_kv, r_k, 128] bf16; cos_table / sin_table fp32 [table_rows >= recon_len, 128];
+ *   out [B, n_q, r_v]; the rest as for palu_flash_decode with recon_len in place of seq_len. r_k a multiple of 32
+ *   (16 when tiled) up to 128. workspace: palu_naive_workspace_bytes, 16-byte aligned. */
+int palu_naive_decode(const void* q, const void* k_latent, const void* u_k, const float* cos_table, const float* sin_table,
+                      int table_rows, const void* v_latent, const int32_t* cur_pos, void* out, float scale, int batch,
+                      int n_q, int n_kv, int seq_len, int recon_len, int r_k, int r_v, int out_dtype, int cache_layout,
+                      int deterministic, void* workspace, size_t workspace_bytes, palu_stream_t stream);
+
+/* Workspace bytes of palu_naive_decode: the rebuilt keys and the flash-decode's split partials (0 for invalid shapes). */
+size_t palu_naive_workspace_bytes(int batch, int n_kv, int recon_len, int r_v);
 
 /* ---- Prefill ----------------------------------------------------------------------------------------
  * The attention of a prefill (the reference's palu_tt/attention.py:380-480 runs it as separate ttnn ops). */

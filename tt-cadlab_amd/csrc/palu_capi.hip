@@ -383,33 +383,6 @@ int sdpa_dispatch(const DecodeArgs& a, bool paged, int cache_layout, int r_k, in
                : dispatch_latent_rows(a, r_k, r_v, cs_dtype, out_dtype, stream);
 }
 
-int flash_setup(DecodeArgs& a, const void* q, const void* k, const void* v, const int32_t* cur_pos, void* out,
-                float scale, int batch, int n_q, int n_kv, int seq_len, int head_dim_v, int out_dtype, int cache_layout,
-                int deterministic, void* workspace, size_t workspace_bytes, const char* who) {
-  if (!q || !k || !v || !cur_pos || !out) return fail(PALU_EINVAL, "%s: a required tensor pointer is null", who);
-  if (batch <= 0 || n_q <= 0 || n_kv <= 0 || seq_len <= 0)
-    return fail(PALU_EINVAL, "%s: batch, head counts and seq_len must be positive", who);
-  if (n_q % n_kv != 0 || n_q / n_kv > 16)
-    return fail(PALU_EINVAL, "KV head count %d must divide the %d query heads with at most 16 query heads per KV head", n_kv, n_q);
-  if (out_dtype != PALU_DTYPE_F32 && out_dtype != PALU_DTYPE_BF16) return fail(PALU_EINVAL, "output dtype must be fp32 or bf16");
-  if (int rc = check_layout(cache_layout, seq_len, who)) return rc;
-  if (!aligned16(q) || !aligned16(k) || !aligned16(v)) return fail(PALU_EINVAL, "q, k and v must be 16-byte aligned");
-  if ((long long)batch * n_kv > 65535) return fail(PALU_EUNSUPPORTED, "batch * n_kv = %d exceeds the grid limit", batch * n_kv);
-  memset(&a, 0, sizeof(a));
-  a.q = static_cast<const __bf16*>(q);
-  a.k = static_cast<const __bf16*>(k);
-  a.v = static_cast<const __bf16*>(v);
-  a.cur_pos = cur_pos;
-  a.out = out;
-  a.ws = static_cast<float*>(workspace);
-  a.ws_bytes = workspace_bytes;
-  a.B = batch; a.n_q = n_q; a.n_kv = n_kv; a.rep = n_q / n_kv; a.hpg = 1; a.S = seq_len; a.cs_rows = 0;
-  a.out_tiled = 0;
-  a.deterministic = deterministic ? 1 : 0;
-  a.qscale = scale * 1.4426950408889634f;
-  return PALU_OK;
-}
-
 // Scratch of palu_sdpa_decode_noalloc: a static device array, one copy per GPU the library runs on. Host
 // code never uses the array's name as an address: its device address comes from hipGetSymbolAddress,
 // once per device with that device current, and is kept per device.
@@ -445,6 +418,33 @@ int scratch_of_current_device(void** addr) {
 }  // namespace
 
 namespace palu {
+
+int flash_setup(DecodeArgs& a, const void* q, const void* k, const void* v, const int32_t* cur_pos, void* out,
+                float scale, int batch, int n_q, int n_kv, int seq_len, int head_dim_v, int out_dtype, int cache_layout,
+                int deterministic, void* workspace, size_t workspace_bytes, const char* who) {
+  if (!q || !k || !v || !cur_pos || !out) return fail(PALU_EINVAL, "%s: a required tensor pointer is null", who);
+  if (batch <= 0 || n_q <= 0 || n_kv <= 0 || seq_len <= 0)
+    return fail(PALU_EINVAL, "%s: batch, head counts and seq_len must be positive", who);
+  if (n_q % n_kv != 0 || n_q / n_kv > 16)
+    return fail(PALU_EINVAL, "KV head count %d must divide the %d query heads with at most 16 query heads per KV head", n_kv, n_q);
+  if (out_dtype != PALU_DTYPE_F32 && out_dtype != PALU_DTYPE_BF16) return fail(PALU_EINVAL, "output dtype must be fp32 or bf16");
+  if (int rc = check_layout(cache_layout, seq_len, who)) return rc;
+  if (!aligned16(q) || !aligned16(k) || !aligned16(v)) return fail(PALU_EINVAL, "q, k and v must be 16-byte aligned");
+  if ((long long)batch * n_kv > 65535) return fail(PALU_EUNSUPPORTED, "batch * n_kv = %d exceeds the grid limit", batch * n_kv);
+  memset(&a, 0, sizeof(a));
+  a.q = static_cast<const __bf16*>(q);
+  a.k = static_cast<const __bf16*>(k);
+  a.v = static_cast<const __bf16*>(v);
+  a.cur_pos = cur_pos;
+  a.out = out;
+  a.ws = static_cast<float*>(workspace);
+  a.ws_bytes = workspace_bytes;
+  a.B = batch; a.n_q = n_q; a.n_kv = n_kv; a.rep = n_q / n_kv; a.hpg = 1; a.S = seq_len; a.cs_rows = 0;
+  a.out_tiled = 0;
+  a.deterministic = deterministic ? 1 : 0;
+  a.qscale = scale * 1.4426950408889634f;
+  return PALU_OK;
+}
 
 int check_qkv_epi(const QkvEpi& e, int batch, int ncols, const void* src, const char* who) {
   if (!src || !e.pos || !e.cos_t || !e.sin_t || !e.q_out) return fail(PALU_EINVAL, "%s: a required pointer is null", who);

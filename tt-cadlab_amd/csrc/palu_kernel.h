@@ -145,6 +145,11 @@ struct QkvEpi {
 // palu_capi.hip; `who` names the entry point in the message).
 int check_qkv_epi(const QkvEpi& e, int batch, int ncols, const void* src, const char* who);
 
+// Checks the operands of a stock flash-decode and fills `a` but for the cache strides (defined in palu_capi.hip).
+int flash_setup(DecodeArgs& a, const void* q, const void* k, const void* v, const int32_t* cur_pos, void* out,
+                float scale, int batch, int n_q, int n_kv, int seq_len, int head_dim_v, int out_dtype, int cache_layout,
+                int deterministic, void* workspace, size_t workspace_bytes, const char* who);
+
 // Waves per workgroup: 8 (two per SIMD) where the kernel fits 256 registers, else 4 (one per SIMD,
 // which lets the compiler use the full 512-entry register file instead of spilling).
 template <int RK, int RV, bool KFULL, bool TILED>

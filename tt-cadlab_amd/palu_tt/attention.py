@@ -263,30 +263,26 @@ class PaluAttention(torch.nn.Module):
 
     def _naive_attention(self, q4, keys, values, pos):
         """The reference's non-fused decode (attention.py:657-710) on the GPU: K = latent @ u_k for the
-        first recon_len positions (bf16 GEMM, fp32 accumulate), Meta RoPE at positions 0..S-1 (the HIP
-        rope kernel), grouped V rebuilt per head with u_v, then the stock flash-decode (the MLA op:
-        V of width r_v for per-head latents, 128 for grouped ones). Returns [1, B, nh, out_width]."""
+        first recon_len positions, Meta RoPE at positions 0..S-1, then the stock flash-decode over them and
+        the V latent (fused.naive_decode); for grouped latents torch GEMMs rebuild K and, with u_v, V per
+        head and the HIP rope kernel rotates K. Returns [1, B, nh, out_width]."""
         S = self._recon_len()
         if self.palu.runtime.check:
             top = int(pos.max())
             assert top < S, f"recon_len {S} does not cover current_pos max {top}"
+        if self.gs == 1:
+            return fused.naive_decode(q4, keys, self.u_k, self.cos, self.sin, values, pos, S, scale=self.scale,
+                                      deterministic=bool(self.palu.runtime.deterministic))
         B, nkv, hd, gs = self.max_batch_size, self.n_kv_heads, self.head_dim, self.gs
-        per_head = lambda lat: lat if gs == 1 else lat.repeat_interleave(gs, dim=1)     # group -> head latents
-        k_lat = per_head(self._cache_rows(keys, S)).contiguous()                          # [B, nkv, S, r_k]
-        k = torch.matmul(k_lat, self.u_k.contiguous())                                    # [B, nkv, S, hd] bf16
+        per_head = lambda lat: lat.repeat_interleave(gs, dim=1).contiguous()              # group -> head latents
+        k = torch.matmul(per_head(self._cache_rows(keys, S)), self.u_k.contiguous())      # [B, nkv, S, hd] bf16
         rows = B * nkv * S
         rpos = self._naive_pos.get(rows)
         if rpos is None:
             rpos = torch.arange(S, dtype=torch.int32, device=self.device).repeat(B * nkv)
             self._naive_pos[rows] = rpos
         k_rot = decoder_ops.rope_rows(k.view(rows, hd), 1, rpos, self.cos, self.sin).view(B, nkv, S, hd)
-        v_lat = self._cache_rows(values, S)
-        if gs > 1:
-            v = torch.matmul(per_head(v_lat).contiguous(), self.u_v.contiguous())          # [B, nkv, S, hd]
-        else:
-            v = v_lat.contiguous()                                                         # absorbed V: [B, nkv, S, r_v]
-        if v.shape[-1] % 32:   # V widths in 16s exist only as tiled caches (16-wide V tiles): hand both over tiled
-            k_rot, v = LatentCache.from_rows(k_rot, "k"), LatentCache.from_rows(v, "v")
+        v = torch.matmul(per_head(self._cache_rows(values, S)), self.u_v.contiguous())    # [B, nkv, S, hd]
         return fused.flash_decode(q4, k_rot, v, pos, scale=self.scale, head_dim_v=self.out_width,
                                   deterministic=bool(self.palu.runtime.deterministic))
 

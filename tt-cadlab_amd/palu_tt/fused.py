@@ -409,6 +409,48 @@ def flash_decode(q, k, v, cur_pos_tensor, *, scale=None, head_dim_v=None, out_dt
     return out
 
 
+def naive_decode(q, k_latent, u_k, cos, sin, v_latent, cur_pos_tensor, recon_len, *, scale=None,
+                 out_dtype=torch.bfloat16, deterministic=False) -> torch.Tensor:
+    """The decode of per-head latents without the fused op: K = RoPE(k_latent @ u_k) is rebuilt for the first
+    recon_len positions (bf16; positions past a row's cur_pos are skipped) and the stock flash-decode runs over it
+    and v_latent. k_latent, v_latent: LatentCache pair or row-major [B, n_kv, S, r] tensors; u_k [n_kv, r_k, 128];
+    cos, sin fp32 [>= recon_len, 128] (cos_sin_tables). Returns [1, B, n_q, r_v]."""
+    if not (isinstance(q, torch.Tensor) and q.dim() == 4 and q.shape[0] == 1 and q.shape[3] == HEAD_DIM):
+        raise RuntimeError(f"q must be [1, B, n_q, {HEAD_DIM}]")
+    dev = q.device
+    _as_dev(q, "q", torch.bfloat16)
+    k_store, k_shape, layout = _cache_arg(k_latent, "k_latent", dev, "k")
+    v_store, v_shape, v_layout = _cache_arg(v_latent, "v_latent", dev, "v")
+    if layout != v_layout:
+        raise RuntimeError("k_latent and v_latent must use the same cache layout")
+    B, n_kv, S, r_k = k_shape
+    if tuple(v_shape[:3]) != (B, n_kv, S):
+        raise RuntimeError(f"v {v_shape} does not match k {k_shape} in [B, n_kv, S]")
+    if q.shape[1] != B:
+        raise RuntimeError(f"q has batch {q.shape[1]} but the caches have {B}")
+    _as_dev(u_k, "u_k", torch.bfloat16, dev)
+    if tuple(u_k.shape) != (n_kv, r_k, HEAD_DIM):
+        raise RuntimeError(f"u_k must be [{n_kv}, {r_k}, {HEAD_DIM}], got {tuple(u_k.shape)}")
+    for t, name in ((cos, "cos"), (sin, "sin")):
+        _as_dev(t, name, torch.float32, dev)
+        if not (t.dim() == 2 and t.shape[1] == HEAD_DIM):
+            raise RuntimeError(f"{name} must be [rows, {HEAD_DIM}]")
+    if out_dtype not in _DTYPES:
+        raise RuntimeError(f"out_dtype must be torch.float32 or torch.bfloat16, got {out_dtype}")
+    cp = _cur_pos(cur_pos_tensor, B, dev)
+    n_q, r_v = q.shape[2], v_shape[3]
+    out = torch.empty(1, B, n_q, r_v, dtype=out_dtype, device=dev)
+    lib = _native.load()
+    need = lib.palu_naive_workspace_bytes(B, n_kv, int(recon_len), r_v)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    _native.check(lib.palu_naive_decode(
+        _native.ptr(q), _native.ptr(k_store), _native.ptr(u_k), _native.ptr(cos), _native.ptr(sin),
+        min(cos.shape[0], sin.shape[0]), _native.ptr(v_store), _native.ptr(cp), _native.ptr(out),
+        float(HEAD_DIM ** -0.5 if scale is None else scale), B, n_q, n_kv, S, int(recon_len), r_k, r_v, _DTYPES[out_dtype],
+        layout, int(bool(deterministic)), _native.ptr(ws), ws.numel(), _native.stream_handle(dev)))
+    return out
+
+
 def scaled_dot_product_attention_decode(q, k, v, cur_pos_tensor, scale=None, **_):
     """Name-compatible alias of the stock decode op (full K and V, head_dim_v = 128)."""
     return flash_decode(q, k, v, cur_pos_tensor, scale=scale)
