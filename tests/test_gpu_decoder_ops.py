@@ -586,3 +586,30 @@ def test_sdpa_decode_tiled_rows_output(gpu, B, S, r_k, r_v, hpg):
     torch.cuda.synchronize()
     assert t.shape == (64, nh * width)
     assert torch.equal(decoder_ops.untile_rows(t, B), a[0].reshape(B, nh * width))
+
+
+@pytest.mark.parametrize("x_tiled", [True, False])
+@pytest.mark.parametrize("rtw,ks", [(1, 1), (2, 4), (3, 1), (4, 2), (5, 1), (6, 1), (7, 1), (8, 4)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33])
+def test_linear_of_few_rows_equals_the_64_row_product(gpu, rows, rtw, ks, x_tiled):
+    """The kernels for up to 16, 32 and 64 rows sum the same products in the same order: the rows of a call of few rows
+    are bit for bit those of a 64-row call, in every output mode that does not write a cache."""
+    g = torch.Generator().manual_seed(rows + rtw)
+    n, k = 16 * 52, 1056
+    x = torch.randn(64, k, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    h = torch.randn(64, n, generator=g).to(torch.bfloat16).cuda()
+    wt = decoder_ops.tile_weight(w, rtw)
+    few, kw = (decoder_ops.tile_rows(x), dict(x_tiled=True, rows=rows)) if x_tiled else (x[:rows], {})
+    for mode in ("bf16", "partials"):
+        full = decoder_ops.linear_tiled(x, wt, rtw, ks, mode=mode)
+        got = decoder_ops.linear_tiled(few, wt, rtw, ks, mode=mode, **kw)
+        assert torch.equal(got, full[:rows] if mode == "bf16" else full[:, :rows]), mode
+    if ks == 1:
+        full = decoder_ops.untile_rows(decoder_ops.linear_tiled(x, wt, rtw, 1, mode="swiglu"), rows)
+        assert torch.equal(decoder_ops.untile_rows(decoder_ops.linear_tiled(few, wt, rtw, 1, mode="swiglu", **kw), rows), full)
+        full = decoder_ops.untile_rows(decoder_ops.linear_swiglu_rmsnorm(x, wt, rtw, 1e-5), rows)
+        assert torch.equal(decoder_ops.untile_rows(decoder_ops.linear_swiglu_rmsnorm(few, wt, rtw, 1e-5, **kw), rows), full)
+        full, ht = decoder_ops.linear_residual(x, wt, rtw, h.clone()), torch.zeros(64, n, dtype=torch.bfloat16, device="cuda")
+        got = decoder_ops.linear_residual(few, wt, rtw, h[:rows].clone(), ht, **kw)
+        assert torch.equal(got, full[:rows]) and torch.equal(decoder_ops.untile_rows(ht, rows), got)

@@ -21,8 +21,8 @@ LIB_NAME = "libpalu_mi355x.so"
 SOURCES = ["palu_capi.hip", "palu_decode_rows.hip", "palu_decode_tiled.hip", "palu_decode_rows_paged.hip",
            "palu_decode_tiled_paged.hip", "palu_decode_tiled_k16.hip", "palu_decode_tiled_paged_k16.hip",
            "palu_decode_full.hip", "palu_glrd.hip", "palu_glrd_narrow.hip", "palu_decoder.hip", "palu_linear.hip",
-           "palu_prefill.hip", "palu_rows.hip", "palu_naive.hip"]
-HEADERS = ["palu_kernel.h", "palu_glrd_scores.h"]
+           "palu_linear_m16.hip", "palu_linear_m32.hip", "palu_prefill.hip", "palu_rows.hip", "palu_naive.hip"]
+HEADERS = ["palu_kernel.h", "palu_glrd_scores.h", "palu_linear_kernel.h"]
 # Per-file flags: the narrow-rank grouped-latent scores kernels keep their MFMA results in VGPRs.
 SOURCE_FLAGS = {"palu_glrd_narrow.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
