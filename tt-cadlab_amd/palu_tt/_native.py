@@ -75,6 +75,8 @@ _lib = None
 def load() -> ctypes.CDLL:
     """The loaded library (loaded once). Raises RuntimeError when it has not been built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -103,4 +105,7 @@ def ptr(t) -> int:
 
 
 def stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of a tensor's device (torch.cuda.current_stream(device).cuda_stream without its Stream object)."""
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)

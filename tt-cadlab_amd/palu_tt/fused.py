@@ -150,19 +150,19 @@ def _grid_cores(program_config) -> Optional[int]:
 _DTYPES = {torch.float32: _native.DTYPE_F32, torch.bfloat16: _native.DTYPE_BF16}
 
 
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def _as_dev(t: torch.Tensor, name: str, dtype=None, device=None) -> torch.Tensor:
-    _require(isinstance(t, torch.Tensor), f"{name} must be a torch.Tensor")
-    _require(t.is_cuda, f"{name} must live on the GPU (got {t.device})")
+    if not isinstance(t, torch.Tensor):
+        raise RuntimeError(f"{name} must be a torch.Tensor")
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must live on the GPU (got {t.device})")
     if device is not None:
-        _require(t.device == device, f"{name} is on {t.device}, expected {device}")
+        if t.device != device:
+            raise RuntimeError(f"{name} is on {t.device}, expected {device}")
     if dtype is not None:
-        _require(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
-    _require(t.is_contiguous(), f"{name} must be contiguous")
+        if t.dtype != dtype:
+            raise RuntimeError(f"{name} must be {dtype}, got {t.dtype}")
+    if not t.is_contiguous():
+        raise RuntimeError(f"{name} must be contiguous")
     return t
 
 
@@ -171,16 +171,17 @@ def _cache_arg(t, name: str, device, role: Optional[str] = None):
     passed where the op reads K (role "k") or V (role "v") must be stored in that role's tile order."""
     if isinstance(t, GroupedLatentCache):
         _as_dev(t.data, name, torch.bfloat16, device)
-        _require(role is not None and t.role == role,
-                 f"{name} is a GroupedLatentCache in {t.role!r} tile order; this argument reads a {role!r} cache")
+        if not (role is not None and t.role == role):
+            raise RuntimeError(f"{name} is a GroupedLatentCache in {t.role!r} tile order; this argument reads a {role!r} cache")
         return t.data, tuple(t.shape), _native.LAYOUT_TILED_GROUPED
     if isinstance(t, LatentCache):
         _as_dev(t.data, name, torch.bfloat16, device)
-        _require(role is None or t.role == role,
-                 f"{name} is a LatentCache in {t.role!r} tile order; this argument reads a {role!r} cache")
+        if not (role is None or t.role == role):
+            raise RuntimeError(f"{name} is a LatentCache in {t.role!r} tile order; this argument reads a {role!r} cache")
         layout = _native.LAYOUT_TILED if t.role == "k" else _native.LAYOUT_TILED_V
         return t.data, tuple(t.shape), (_native.LAYOUT_TILED if role is not None else layout)
-    _require(isinstance(t, torch.Tensor) and t.dim() == 4, f"{name} must be [B, n_groups, S, width] or a LatentCache")
+    if not (isinstance(t, torch.Tensor) and t.dim() == 4):
+        raise RuntimeError(f"{name} must be [B, n_groups, S, width] or a LatentCache")
     _as_dev(t, name, torch.bfloat16, device)
     return t, tuple(t.shape), _native.LAYOUT_ROWS
 
@@ -190,8 +191,8 @@ def _workspace(batch: int, n_kv: int, seq_len: int, width: int, device, workspac
     if need == 0:
         return None, 0
     if workspace is not None:
-        _require(workspace.is_cuda and workspace.numel() * workspace.element_size() >= need,
-                 f"workspace must hold {need} bytes on the GPU")
+        if not (workspace.is_cuda and workspace.numel() * workspace.element_size() >= need):
+            raise RuntimeError(f"workspace must hold {need} bytes on the GPU")
         return workspace, workspace.numel() * workspace.element_size()
     return torch.empty(need, dtype=torch.uint8, device=device), need
 
@@ -200,26 +201,28 @@ def _glrd_workspace(batch: int, n_q: int, n_kv: int, n_groups: int, seq_len: int
     """Workspace of the grouped-latent path: partial scores and latent PV partials between its passes."""
     need = _native.load().palu_glrd_workspace_bytes(batch, n_q, n_kv, n_groups, seq_len, r_v)
     if workspace is not None:
-        _require(workspace.is_cuda and workspace.numel() * workspace.element_size() >= need,
-                 f"workspace must hold {need} bytes on the GPU (palu_glrd_workspace_bytes)")
+        if not (workspace.is_cuda and workspace.numel() * workspace.element_size() >= need):
+            raise RuntimeError(f"workspace must hold {need} bytes on the GPU (palu_glrd_workspace_bytes)")
         return workspace, workspace.numel() * workspace.element_size()
     return torch.empty(max(need, 1), dtype=torch.uint8, device=device), need
 
 
 def _cur_pos(cur_pos_tensor: torch.Tensor, batch: int, device) -> torch.Tensor:
-    _require(isinstance(cur_pos_tensor, torch.Tensor), "cur_pos_tensor must be a torch.Tensor")
+    if not isinstance(cur_pos_tensor, torch.Tensor):
+        raise RuntimeError("cur_pos_tensor must be a torch.Tensor")
     cp = cur_pos_tensor.reshape(-1)
-    _require(cp.numel() == batch, f"cur_pos_tensor has {cp.numel()} entries for batch {batch}")
+    if cp.numel() != batch:
+        raise RuntimeError(f"cur_pos_tensor has {cp.numel()} entries for batch {batch}")
     if cp.device != device or cp.dtype != torch.int32:
         cp = cp.to(device=device, dtype=torch.int32)
     return cp.contiguous()
 
 
 def _page_table(page_table_tensor, batch: int, device) -> torch.Tensor:
-    _require(isinstance(page_table_tensor, torch.Tensor) and page_table_tensor.dim() == 2,
-             "page_table_tensor must be [B, max_pages_per_seq] int32")
-    _require(page_table_tensor.shape[0] == batch,
-             f"page_table_tensor has {page_table_tensor.shape[0]} rows for batch {batch}")
+    if not (isinstance(page_table_tensor, torch.Tensor) and page_table_tensor.dim() == 2):
+        raise RuntimeError("page_table_tensor must be [B, max_pages_per_seq] int32")
+    if page_table_tensor.shape[0] != batch:
+        raise RuntimeError(f"page_table_tensor has {page_table_tensor.shape[0]} rows for batch {batch}")
     pt = page_table_tensor
     if pt.device != device or pt.dtype != torch.int32:
         pt = pt.to(device=device, dtype=torch.int32)
@@ -231,11 +234,12 @@ def _pool_dims(k_shape, v_shape, q, page_table_tensor, dev, what):
     [B, G, S, r] or paged pools [n_pages, G, page_size, r] with a [B, max_pages] page table."""
     if page_table_tensor is None:
         B, G, S, r_k = k_shape
-        _require(tuple(v_shape[:3]) == (B, G, S), f"v {v_shape} does not match k {k_shape} in [B, {what}, S]")
+        if tuple(v_shape[:3]) != (B, G, S):
+            raise RuntimeError(f"v {v_shape} does not match k {k_shape} in [B, {what}, S]")
         return B, G, S, r_k, v_shape[3], None, 0, 0
     n_pages, G, page_size, r_k = k_shape
-    _require(tuple(v_shape[:3]) == (n_pages, G, page_size),
-             f"v pool {v_shape} does not match k pool {k_shape} in [n_pages, {what}, page_size]")
+    if tuple(v_shape[:3]) != (n_pages, G, page_size):
+        raise RuntimeError(f"v pool {v_shape} does not match k pool {k_shape} in [n_pages, {what}, page_size]")
     B = q.shape[1]
     pt = _page_table(page_table_tensor, B, dev)
     return B, G, pt.shape[1] * page_size, r_k, v_shape[3], pt, page_size, n_pages
@@ -272,26 +276,31 @@ def palu_sdpa_decode(q, k_latent, w_rot, cs_tab, v_latent, head_dim_v, cur_pos_t
     device memory at all (for HIP graph capture and serving loops); calls overlapping on one GPU race.
     """
     del compute_kernel_config, memory_config
-    _require(isinstance(q, torch.Tensor) and q.dim() == 4 and q.shape[0] == 1 and q.shape[3] == HEAD_DIM,
-             f"q must be [1, B, n_q, {HEAD_DIM}], got {tuple(getattr(q, 'shape', ()))}")
+    if not (isinstance(q, torch.Tensor) and q.dim() == 4 and q.shape[0] == 1 and q.shape[3] == HEAD_DIM):
+        raise RuntimeError(f"q must be [1, B, n_q, {HEAD_DIM}], got {tuple(getattr(q, 'shape', ()))}")
     dev = q.device
     _as_dev(q, "q", torch.bfloat16)
     k_store, k_shape, layout = _cache_arg(k_latent, "k_latent", dev, "k")
     v_store, v_shape, v_layout = _cache_arg(v_latent, "v_latent", dev, "v")
-    _require(layout == v_layout, "k_latent and v_latent must use the same cache layout")
+    if layout != v_layout:
+        raise RuntimeError("k_latent and v_latent must use the same cache layout")
     B, n_groups, S, r_k, r_v, pt, page_size, n_pages = _pool_dims(k_shape, v_shape, q, page_table_tensor, dev,
                                                                  "n_groups")
-    _require(q.shape[1] == B, f"q has batch {q.shape[1]} but the latent caches have {B}")
+    if q.shape[1] != B:
+        raise RuntimeError(f"q has batch {q.shape[1]} but the latent caches have {B}")
     n_q = q.shape[2]
     w = w_rot.reshape(-1, *w_rot.shape[-2:]) if w_rot.dim() >= 3 else w_rot
-    _require(w.dim() == 3 and (w_rot.dim() == 3 or w_rot.shape[0] == 1),
-             f"w_rot must be [1, n_kv, r_k, 256], got {tuple(w_rot.shape)}")
+    if not (w.dim() == 3 and (w_rot.dim() == 3 or w_rot.shape[0] == 1)):
+        raise RuntimeError(f"w_rot must be [1, n_kv, r_k, 256], got {tuple(w_rot.shape)}")
     _as_dev(w, "w_rot", torch.bfloat16, dev)
     n_kv, w_rank, w_width = w.shape
-    _require(w_rank == r_k, f"w_rot rank {w_rank} != k_latent width r_k {r_k}")
+    if w_rank != r_k:
+        raise RuntimeError(f"w_rot rank {w_rank} != k_latent width r_k {r_k}")
     cs = cs_tab.reshape(-1, cs_tab.shape[-1])
-    _require(cs_tab.dim() in (2, 4), f"cs_tab must be [1, 1, S, 256], got {tuple(cs_tab.shape)}")
-    _require(cs.dtype in (torch.float32, torch.bfloat16), f"cs_tab must be fp32 or bf16, got {cs.dtype}")
+    if cs_tab.dim() not in (2, 4):
+        raise RuntimeError(f"cs_tab must be [1, 1, S, 256], got {tuple(cs_tab.shape)}")
+    if cs.dtype not in (torch.float32, torch.bfloat16):
+        raise RuntimeError(f"cs_tab must be fp32 or bf16, got {cs.dtype}")
     _as_dev(cs, "cs_tab", None, dev)
     rot = ROT_MODES.get(rot_mode, -1) if isinstance(rot_mode, str) else -1
     if rot < 0:
@@ -301,8 +310,9 @@ def palu_sdpa_decode(q, k_latent, w_rot, cs_tab, v_latent, head_dim_v, cur_pos_t
         hpg = n_kv // n_groups if n_groups and n_kv % n_groups == 0 else 1
         if cores is not None and hpg > 1 and int(heads_per_core) <= n_kv and hpg % int(heads_per_core) == 0:
             items = B * (n_kv // int(heads_per_core))
-            _require(items <= cores, f"heads_per_core={heads_per_core} needs {items} cores for {B} rows of "
-                                     f"{n_kv // int(heads_per_core)} head groups, only {cores} available")
+            if items > cores:
+                raise RuntimeError(f"heads_per_core={heads_per_core} needs {items} cores for {B} rows of "
+                                   f"{n_kv // int(heads_per_core)} head groups, only {cores} available")
     if out_dtype not in _DTYPES:
         raise RuntimeError(f"out_dtype must be torch.float32 or torch.bfloat16, got {out_dtype}")
     cp = _cur_pos(cur_pos_tensor, B, dev)
@@ -312,34 +322,39 @@ def palu_sdpa_decode(q, k_latent, w_rot, cs_tab, v_latent, head_dim_v, cur_pos_t
     width = int(head_dim_v)
     od = _DTYPES[out_dtype]
     if tiled_rows:
-        _require(out_dtype == torch.bfloat16 and B <= 64, "a tiled-rows output is bf16 for at most 64 rows")
+        if not (out_dtype == torch.bfloat16 and B <= 64):
+            raise RuntimeError("a tiled-rows output is bf16 for at most 64 rows")
         od |= _native.OUT_TILED_ROWS
         if out is None:
             out = torch.empty(64, n_q * width, dtype=out_dtype, device=dev)
         _as_dev(out, "out", out_dtype, dev)
-        _require(tuple(out.shape) == (64, n_q * width) and out.is_contiguous(), f"out must be [64, {n_q * width}]")
+        if not (tuple(out.shape) == (64, n_q * width) and out.is_contiguous()):
+            raise RuntimeError(f"out must be [64, {n_q * width}]")
     elif out is None:
         out = torch.empty(1, B, n_q, width, dtype=out_dtype, device=dev)
     else:
         _as_dev(out, "out", out_dtype, dev)
-        _require(tuple(out.shape) == (1, B, n_q, width), f"out must be [1, {B}, {n_q}, {width}]")
+        if tuple(out.shape) != (1, B, n_q, width):
+            raise RuntimeError(f"out must be [1, {B}, {n_q}, {width}]")
     gr = None
     if layout == _native.LAYOUT_TILED_GROUPED:
         # compact grouped caches carry their groups' ranks; group_ranks, when given, must agree
         cache_ranks = [list(k_latent.ranks), list(v_latent.ranks)]
-        _require(group_ranks is None or [[int(r) for r in x] for x in group_ranks] == cache_ranks,
-                 f"group_ranks {group_ranks} differ from the GroupedLatentCache ranks {cache_ranks}")
+        if not (group_ranks is None or [[int(r) for r in x] for x in group_ranks] == cache_ranks):
+            raise RuntimeError(f"group_ranks {group_ranks} differ from the GroupedLatentCache ranks {cache_ranks}")
         group_ranks = cache_ranks
     if group_ranks is not None:
         gk, gv = (list(x) for x in group_ranks)
-        _require(len(gk) == n_groups and len(gv) == n_groups,
-                 f"group_ranks must give {n_groups} K ranks and {n_groups} V ranks")
-        _require(pt is None, "group_ranks: per-group ranks are built for contiguous caches")
+        if not (len(gk) == n_groups and len(gv) == n_groups):
+            raise RuntimeError(f"group_ranks must give {n_groups} K ranks and {n_groups} V ranks")
+        if pt is not None:
+            raise RuntimeError("group_ranks: per-group ranks are built for contiguous caches")
         gr = (ctypes.c_int32 * (2 * n_groups))(*[int(r) for r in gk + gv])
     lib = _native.load()
     sc = float(HEAD_DIM ** -0.5 if scale is None else scale)
     if noalloc:
-        _require(pt is None and workspace is None, "noalloc takes contiguous caches and no workspace")
+        if not (pt is None and workspace is None):
+            raise RuntimeError("noalloc takes contiguous caches and no workspace")
         _native.check(lib.palu_sdpa_decode_noalloc(
             _native.ptr(q), _native.ptr(k_store), _native.ptr(w), _native.ptr(cs), _native.ptr(v_store), width,
             _native.ptr(cp), _native.ptr(out), _native.ptr(rs), _native.ptr(tm), _native.ptr(uv), gr, sc,
@@ -375,18 +390,22 @@ def flash_decode(q, k, v, cur_pos_tensor, *, scale=None, head_dim_v=None, out_dt
     flash_multi_latent_attention_decode (head_dim_v = V width). Returns [1, B, n_q, head_dim_v].
     With page_table_tensor, k and v are page pools [n_pages, n_kv, page_size, width] (ttnn's
     paged_scaled_dot_product_attention_decode)."""
-    _require(isinstance(q, torch.Tensor) and q.dim() == 4 and q.shape[0] == 1 and q.shape[3] == HEAD_DIM,
-             f"q must be [1, B, n_q, {HEAD_DIM}]")
+    if not (isinstance(q, torch.Tensor) and q.dim() == 4 and q.shape[0] == 1 and q.shape[3] == HEAD_DIM):
+        raise RuntimeError(f"q must be [1, B, n_q, {HEAD_DIM}]")
     dev = q.device
     _as_dev(q, "q", torch.bfloat16)
     k_store, k_shape, layout = _cache_arg(k, "k", dev, "k")
     v_store, v_shape, v_layout = _cache_arg(v, "v", dev, "v")
-    _require(layout == v_layout, "k and v must use the same cache layout")
+    if layout != v_layout:
+        raise RuntimeError("k and v must use the same cache layout")
     B, n_kv, S, hd, v_width, pt, page_size, n_pages = _pool_dims(k_shape, v_shape, q, page_table_tensor, dev, "n_kv")
-    _require(hd == HEAD_DIM, f"k must be [B, n_kv, S, {HEAD_DIM}], got {k_shape}")
-    _require(q.shape[1] == B, f"q has batch {q.shape[1]} but the caches have {B}")
+    if hd != HEAD_DIM:
+        raise RuntimeError(f"k must be [B, n_kv, S, {HEAD_DIM}], got {k_shape}")
+    if q.shape[1] != B:
+        raise RuntimeError(f"q has batch {q.shape[1]} but the caches have {B}")
     width = int(v_width if head_dim_v is None else head_dim_v)
-    _require(width == v_width, f"head_dim_v {width} != V width {v_width}")
+    if width != v_width:
+        raise RuntimeError(f"head_dim_v {width} != V width {v_width}")
     n_q = q.shape[2]
     if out_dtype not in _DTYPES:
         raise RuntimeError(f"out_dtype must be torch.float32 or torch.bfloat16, got {out_dtype}")
@@ -473,7 +492,8 @@ def paged_update_cache(cache, new_rows: torch.Tensor, update_idxs_tensor: torch.
     page pool [n_pages, G, page_size, width] and row b goes to page page_table[b, idx // page_size]."""
     dev = cache.device
     if isinstance(cache, GroupedLatentCache):
-        _require(page_table is None, "a GroupedLatentCache is contiguous")
+        if page_table is not None:
+            raise RuntimeError("a GroupedLatentCache is contiguous")
         B, G, S, width = cache.shape
         decoder_ops.append_from(cache, new_rows.reshape(B, G * width), width, width, update_idxs_tensor)
         return
