@@ -8,18 +8,20 @@
 //      accumulation), and V: the latent rows themselves where V stays latent, or lat u_v in fp32;
 //   3. palu_prefill_attn_kernel: flash attention.
 //
-// Precision on the bf16 matrix cores. An fp32 value x is the sum of three bf16 planes h + m + l (h = bf16(x), m =
-// bf16(x - h), l = bf16(x - h - m): 24 bits, and bf16 has fp32's range, so nothing saturates). A product
-// of two fp32 operands is six MFMAs, hh + hm + mh + mm + hl + lh, dropping terms below 2^-24 of the product; a
-// product with an operand that is exactly bf16 (a V latent, u_v) is three. All sums are fp32. Measured
-// against 64 bits (tests/test_gpu_prefill.py states the bound), the result before its bf16 rounding is closer
-// than the fp32 SDPA chain it replaces (5e-7 relative).
+// Precision on 16-bit matrix cores. Scores: q and K are each the sum of two fp16 planes of their value over a power-of-two
+// scale (plane_scale: one per query row and one per 32-key record, applied again in the exponent), 22 bits, and a
+// product is three MFMAs, hm + mh + hh. Probabilities (and a rebuilt V) are the sum of three bf16 planes h + m + l (24
+// bits, and bf16 has fp32's range); with a V latent, which is exactly bf16, a product is three MFMAs, between two such
+// sums six (terms below 2^-24 dropped). All sums are fp32. Measured against 64 bits over 17 to 4096 positions, ranks 32 to
+// 512 and scores of spread 1 and 4, the result before its bf16 rounding is off by 2.3e-7 to 1.06e-6 (relative 2-norm);
+// with three bf16 planes and six MFMAs for the scores as well it is 2.5e-7 to 1.29e-6 (twice as many fp32 additions),
+// and the fp32 SDPA chain that the kernels replace 3.3e-7 to 1.76e-6.
 //
 // With per-head latents V is never rebuilt: softmax(q K^T) (v_lat u_v) = (softmax(q K^T) v_lat) u_v, so the
 // probabilities multiply the bf16 latent rows (three MFMAs over r_v columns instead of six over 128) and u_v
 // is applied once per query at the end.
 //
-// Bound: MFMA. Per query head and (query, key) pair 6 x 128 + 3 x r_v multiply-adds.
+// Per query head and (query, key) pair 3 x 128 + 3 x r_v multiply-adds.
 #include "palu_kernel.h"
 
 #include <algorithm>
@@ -27,7 +29,7 @@
 namespace {
 
 constexpr int PF_ROWS = 256;              // query rows (position, head of the KV group) per workgroup
-constexpr int PF_KTILES = 24;             // K tiles of a 32-key record: 3 planes x 2 half-blocks x 4 dim blocks
+constexpr int PF_KTILES = 16;             // K tiles of a 32-key record: 2 planes x 2 half-blocks x 4 dim blocks
 
 struct PrefillArgs {
   const __bf16* x;                        // QKV projection rows [U * S][ldx]
@@ -41,7 +43,8 @@ struct PrefillArgs {
   const float* sin_t;
   int table_rows;
   float qscale;                           // softmax scale * log2 e
-  __bf16* rec;                            // records [U * nkv][nblk][tiles][64][8]
+  __bf16* rec;                            // records [U * nkv][nblk][tiles][64][8] (K tiles fp16, V tiles bf16)
+  float* ksc;                             // power-of-two scale of a record's K planes [U * nkv][nblk]
   __bf16* uvt;                            // u_v^T tiles [nkv][KBV][8][64][8] (up-projection)
   __bf16* out;                            // [U * S][ldo]
   long long ldo;
@@ -67,12 +70,31 @@ __device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8& h, bf16x8&
   }
 }
 
+// x = s (h + m) with fp16 planes h, m of x / s: s a power of two that puts the largest magnitude of the set that x belongs
+// to (amax) in [2^14, 2^15), so that no value saturates and the planes hold 22 bits of every value above amax 2^-17 (and an
+// absolute 2^-39 amax of the rest). A zero or non-finite amax gives s = 2^-15 (non-finite values stay so); s is at least
+// 2^-63, so that a product of two scales is a normal number.
+__device__ __forceinline__ float plane_scale(float amax, float& inv) {
+  const int e = max(-48, min(126, __builtin_amdgcn_frexp_expf(amax))) - 15;
+  inv = __builtin_amdgcn_ldexpf(1.f, -e);
+  return __builtin_amdgcn_ldexpf(1.f, e);
+}
+
+__device__ __forceinline__ void split2x8(const float (&v)[8], float inv, f16x8& h, f16x8& m) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float y = v[j] * inv;
+    h[j] = (_Float16)y;
+    m[j] = (_Float16)(y - (float)h[j]);
+  }
+}
+
 // Position of operand column nn of half-block c of a 32-position block (the K-tile order of the caches): the
 // scores of tile c then leave lane (n, g) with keys 8 g + 4 c .. + 3, so the two tiles together are the eight
 // consecutive keys of the PV product's operand.
 __device__ __forceinline__ int blk_pos(int nn, int c) { return 8 * (nn >> 2) + 4 * c + (nn & 3); }
 
-// Records of one (user, KV head, 32-position block): K planes as MFMA operand tiles [plane][c][kb] (lane (n, g) of
+// Records of one (user, KV head, 32-position block): fp16 K planes as MFMA operand tiles [plane][c][kb] (lane (n, g) of
 // tile (c, kb) holds dims 32 kb + {4 g .. + 3, 16 + 4 g .. + 3} of position blk_pos(n, c)) and V tiles behind them
 // (tile mt, lane (m, g): positions 8 g .. + 7 of column 16 mt + m; three planes of 8 tiles when V is rebuilt).
 // Positions past the prompt are zero. blockIdx.y 0 writes K, 1 writes V; a wave takes one block. u_k / u_v go
@@ -179,33 +201,46 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
     }
   }
   if (!live) return;
-  bf16x8 h, m, l;
   if (!isv) {
     // lane (n, g), tile c: dims 16 t + 4 g + i of position blk_pos(n, c); two tiles make one operand slot
+    float amax = 0.f;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int pr = min(p[c], a.table_rows - 1);
 #pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        float q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = acc[c][t][i];
+        rope_meta<4>(q, a.cos_t, a.sin_t, pr, 16 * t + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[c][t][i] = q[i];
+          amax = fmaxf(amax, fabsf(q[i]));
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    float inv;
+    const float sc = plane_scale(amax, inv);
+    if (lane == 0) a.ksc[(long long)uk * a.nblk + jb] = sc;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
         float v[8];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-          float q[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) q[i] = acc[c][2 * kb + hh][i];
-          rope_meta<4>(q, a.cos_t, a.sin_t, pr, 16 * (2 * kb + hh) + 4 * g);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[4 * hh + i] = q[i];
-        }
-        split3x8(v, h, m, l);
+        for (int i = 0; i < 8; ++i) v[i] = acc[c][2 * kb + (i >> 2)][i & 3];
+        f16x8 h, m;
+        split2x8(v, inv, h, m);
         __bf16* o = rec + ((c * 4 + kb) * 64 + lane) * 8;
-        *reinterpret_cast<bf16x8*>(o) = h;
-        *reinterpret_cast<bf16x8*>(o + 8 * 512) = m;
-        *reinterpret_cast<bf16x8*>(o + 16 * 512) = l;
+        *reinterpret_cast<f16x8*>(o) = h;
+        *reinterpret_cast<f16x8*>(o + 8 * 512) = m;
       }
-    }
   } else {
     // lane (n, g), tile t: column 16 t + n at positions 8 g + 4 c + i
+    bf16x8 h, m, l;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       float v[8];
@@ -224,7 +259,7 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
 
 // Flash attention over the records. A workgroup owns PF_ROWS rows of one (user, KV head), a row being one
 // (position, query head of the group) in position-major order, so the group's heads share every K and V tile. A
-// wave owns NG column groups of 16 rows; its rotated, scaled query sits in registers as three planes. Each 32-key
+// wave owns NG column groups of 16 rows; its rotated, scaled query sits in registers as two planes. Each 32-key
 // record is copied to LDS once per workgroup (double buffered: the next one's loads are in flight during the
 // arithmetic) and every K tile read from LDS feeds up to 3 NG MFMAs. Scores are computed transposed
 // (keys x rows), so a lane holds eight keys of one row per column group: softmax in the exp2 domain with a lazily
@@ -250,7 +285,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
   const int row0 = qb * PF_ROWS + w * 16 * NG;
 
   int pos[NG];
-  bf16x8 q[3][NG][4];
+  f16x8 q[2][NG][4];
+  float qsc[NG];
 #pragma unroll
   for (int gr = 0; gr < NG; ++gr) {
     const int row = min(row0 + 16 * gr + n, rows - 1);     // rows past the prompt repeat its last one, unstored
@@ -258,9 +294,9 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
     const int head = kvh * a.rep + (row - pos[gr] * a.rep);
     const __bf16* xq = a.x + ((long long)u * a.S + pos[gr]) * a.ldx + (long long)head * HD;
     const int pr = min(pos[gr], a.table_rows - 1);
+    float v[4][8], amax = 0.f;
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      float v[8];
+    for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         const int d = 16 * (2 * kb + hh) + 4 * g;
@@ -270,10 +306,15 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
         for (int i = 0; i < 4; ++i) t[i] = (float)xv[i];
         rope_meta<4>(t, a.cos_t, a.sin_t, pr, d);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[4 * hh + i] = t[i] * a.qscale;
+        for (int i = 0; i < 4; ++i) {
+          v[kb][4 * hh + i] = t[i] * a.qscale;
+          amax = fmaxf(amax, fabsf(v[kb][4 * hh + i]));
+        }
       }
-      split3x8(v, q[0][gr][kb], q[1][gr][kb], q[2][gr][kb]);
-    }
+    float inv;
+    qsc[gr] = plane_scale(wave_max_xor48(amax), inv);       // over the row's four lanes
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) split2x8(v[kb], inv, q[0][gr][kb], q[1][gr][kb]);
   }
   // Keys this wave and this workgroup need; rows are position-major, so the first and last rows bound the wave.
   const int w_lo = min(row0, rows - 1) / a.rep, w_hi = min(row0 + 16 * NG - 1, rows - 1) / a.rep;
@@ -309,6 +350,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
     const int base = j * BLK;
     if (base <= w_hi) {                                     // uniform per wave
       const bf16x8* kt = lds + (j & 1) * NT * 64 + lane;
+      const float ksc = load_uniform_f(a.ksc, (long long)uk * a.nblk + j);
       f32x4 s[NG][2];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
@@ -316,13 +358,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
         for (int gr = 0; gr < NG; ++gr) s[gr][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
-          const bf16x8 kh = kt[(c * 4 + kb) * 64], km = kt[(8 + c * 4 + kb) * 64], kl = kt[(16 + c * 4 + kb) * 64];
-#pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(kl, q[0][gr][kb], s[gr][c]);
-#pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(kh, q[2][gr][kb], s[gr][c]);
-#pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(km, q[1][gr][kb], s[gr][c]);
+          const f16x8 kh = __builtin_bit_cast(f16x8, kt[(c * 4 + kb) * 64]);
+          const f16x8 km = __builtin_bit_cast(f16x8, kt[(8 + c * 4 + kb) * 64]);
 #pragma unroll
           for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(km, q[0][gr][kb], s[gr][c]);
 #pragma unroll
@@ -340,11 +377,12 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
             for (int i = 0; i < 4; ++i)
               if (base + 8 * g + 4 * c + i > pos[gr]) s[gr][c][i] = NEG_INF;
       }
-      float bm[NG];
+      float f[NG], bm[NG];                                  // the planes' scales go into the exponent
       bool up = false;
 #pragma unroll
       for (int gr = 0; gr < NG; ++gr) {
-        bm[gr] = max8(s[gr][0], s[gr][1]);
+        f[gr] = qsc[gr] * ksc;
+        bm[gr] = max8(s[gr][0], s[gr][1]) * f[gr];
         up = up || bm[gr] > m_run[gr] + LAZY_RESCALE_LOG2;
       }
       if (__any(up)) {
@@ -366,7 +404,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) p[4 * c + i] = __builtin_amdgcn_exp2f(s[gr][c][i] - mref);
+          for (int i = 0; i < 4; ++i) p[4 * c + i] = __builtin_amdgcn_exp2f(fmaf(s[gr][c][i], f[gr], -mref));
         l_run[gr] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         split3x8(p, ph[gr], pm[gr], pl[gr]);
       }
@@ -540,8 +578,8 @@ bool prefill_shape_ok(int users, int seq, int n_heads, int n_kv, int n_groups, i
 
 extern "C" size_t palu_prefill_workspace_bytes(int users, int seq, int n_heads, int n_kv, int n_groups, int r_k, int r_v) {
   if (!prefill_shape_ok(users, seq, n_heads, n_kv, n_groups, r_k, r_v)) return 0;
-  const size_t rec = (size_t)users * n_kv * ((seq + 31) / 32) * (PF_KTILES + v_tiles(n_kv, n_groups, r_v)) * 1024;
-  return rec + (size_t)n_kv * 4 * 8 * 1024;
+  const size_t blocks = (size_t)users * n_kv * ((seq + 31) / 32);
+  return blocks * (PF_KTILES + v_tiles(n_kv, n_groups, r_v)) * 1024 + (size_t)n_kv * 4 * 8 * 1024 + blocks * sizeof(float);
 }
 
 extern "C" int palu_prefill_attention(const void* qkv, long long ld, int users, int seq, int n_heads, int n_kv, int n_groups,
@@ -598,7 +636,9 @@ extern "C" int palu_prefill_attention(const void* qkv, long long ld, int users, 
   const bool split = !(per_head && r_v <= HD);
   a.tiles = PF_KTILES + v_tiles(n_kv, n_groups, r_v);
   a.rec = static_cast<__bf16*>(workspace);
-  a.uvt = (split || !u_v) ? nullptr : a.rec + (size_t)users * n_kv * a.nblk * a.tiles * 512;
+  __bf16* uvt = a.rec + (size_t)users * n_kv * a.nblk * a.tiles * 512;
+  a.uvt = (split || !u_v) ? nullptr : uvt;
+  a.ksc = reinterpret_cast<float*>(uvt + (size_t)n_kv * 4 * 8 * 512);
   const dim3 grid((unsigned)(users * n_kv * ((a.nblk + 3) / 4)), 2);
   if (split) hipLaunchKernelGGL(palu_prefill_rebuild_kernel<true>, grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL(palu_prefill_rebuild_kernel<false>, grid, dim3(256), 0, stream, a);
