@@ -105,17 +105,31 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
     }
   };
   auto stage = [&](const bf16x8* cur, bf16x8* nxt, int j, int s) __attribute__((always_inline)) {
+    // The stage's activation tiles in pairs, each pair read from LDS while the one before it is multiplied (left to the
+    // compiler every read stood right before its use), and the products ahead of the other workgroup's address work: 2048 x
+    // 28672 x 4096 434 -> 427 us, 2048 x 4096 x 14336 223 -> 220.
+    bf16x8 b[2][2];
+    auto read = [&](int q) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) b[q & 1][i] = cur[(2 * q + i) * 64 + lane];
+    };
+    read(0);
     load_x(nxt, s + XS - 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int kth = 0; kth < 2; ++kth) {
+    for (int q = 0; q < MT; ++q) {        // k tile q / (MT / 2), row tiles 2 q % MT and the next
+      const int kth = q / (MT / 2);
+      if (q + 1 < MT) read(q + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const bf16x8 b = cur[(kth * MT + t) * 64 + lane];
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) acc[i][t] = mfma16(wr[j % WS][kth][i], b, acc[i][t]);
-      }
-      load_w(j % WS, kth, s + WS);
+        for (int i = 0; i < RPW; ++i)
+          acc[i][(2 * q + h) % MT] = mfma16(wr[j % WS][kth][i], b[q & 1][h], acc[i][(2 * q + h) % MT]);
+      __builtin_amdgcn_s_setprio(0);
+      if (q % (MT / 2) == MT / 2 - 1) load_w(j % WS, kth, s + WS);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // Loads complete in order. The next stage's activations were asked for XS - 2 stages ago and its weights WS - 1
     // stages ago, so once no more than the loads of that many stages are outstanding, both have arrived, and past the
