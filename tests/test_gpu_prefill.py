@@ -84,6 +84,31 @@ def test_prefill_attention_wide_range(gpu):
     assert bool(torch.isfinite(out).all()) and ((out - exp).abs() / bound).max().item() <= 1.0
 
 
+@pytest.mark.parametrize("kf,qf,spike", [(0.0, 1.0, 1.0), (1e-25, 1e22, 1.0), (1e-12, 1e12, 1.0), (1.0, 1.0, 4096.0)])
+def test_prefill_attention_plane_scales(gpu, kf, qf, spike):
+    """The power-of-two scales of the score planes: keys that are all zero, keys and queries far apart in magnitude, and
+    records whose keys differ by 2^12 (position 40's latent large, its products with the query kept small by it)."""
+    x, k0, v0, u_k, u_v, cos, sin = _inputs(1, 96, 8, 2, 2, 64, 64, 9)
+    x = x.clone()
+    x[:, k0:v0] *= kf
+    x[:, :k0] *= qf
+    x[40, k0:v0] *= spike
+    x[:, :k0] /= spike
+    out = decoder_ops.prefill_attention(x, 1, 8, 2, 2, k0, 64, u_k, v0, 64, u_v, cos, sin, HD ** -0.5).double()
+    exp = _exact(x, 1, 8, 2, 2, k0, 64, u_k, v0, 64, u_v, cos, sin, HD ** -0.5)
+    bound = _half_step(exp) * 1.001 + 4e-6 * exp.abs().amax(-1, keepdim=True)
+    assert ((out - exp).abs() / bound).max().item() <= 1.0
+
+
+def test_prefill_whole_v_heads_keep_a_nonfinite_value_in_its_column(gpu):
+    x, k0, v0, u_k, _, cos, sin = _inputs(1, 64, 4, 1, 1, 64, HD, 3, full_v=True)
+    x = x.clone()
+    x[50, v0 + 21] = float("inf")
+    out = decoder_ops.prefill_attention(x, 1, 4, 1, 1, k0, 64, u_k, v0, HD, None, cos, sin, HD ** -0.5)
+    other = torch.arange(4 * HD, device="cuda") % HD != 21
+    assert bool(torch.isfinite(out[:, other]).all()) and not bool(torch.isfinite(out[50:, ~other]).any())
+
+
 @pytest.mark.parametrize("kind,w", [("rows", 40), ("rows", 64), ("k", 48), ("k", 64), ("k", 112), ("v", 16), ("v", 80)])
 @pytest.mark.parametrize("n_pos", [1, 8, 37, 64])
 def test_fill_matches_write_rows(gpu, kind, w, n_pos):

@@ -51,6 +51,18 @@ struct PrefillArgs {
   int nblk, tiles;
 };
 
+// rope_meta of four values, the table read in 16 bytes (its columns come in equal pairs).
+__device__ __forceinline__ void rope4(float (&v)[4], const float* cos_t, const float* sin_t, int pr, int c) {
+  const f32x4 cs = *reinterpret_cast<const f32x4*>(cos_t + (long long)pr * HD + c);
+  const f32x4 sn = *reinterpret_cast<const f32x4*>(sin_t + (long long)pr * HD + c);
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    const float x0 = v[i], x1 = v[i + 1];
+    v[i] = fmaf(x0, cs[i], -(x1 * sn[i]));
+    v[i + 1] = fmaf(x1, cs[i], x0 * sn[i]);
+  }
+}
+
 // x = h + m + l in bf16 planes.
 __device__ __forceinline__ void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
   h = (__bf16)x;
@@ -118,9 +130,8 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
   const int grp = kvh / a.hpg;
 
   if (isv && !VSPLIT) {                   // V stays latent: a transposing copy, and u_v^T for the up-projection
-    const int vt = a.r_v >> 4;
-    if (live) {
-      for (int mt = 0; mt < vt; ++mt) {
+    if (live && !a.u_v) {                 // whole V heads: element by element, so that a non-finite value stays in its column
+      for (int mt = 0; mt < 8; ++mt) {
         bf16x8 o;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -128,6 +139,40 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
           const __bf16 v = xu[(long long)min(p, a.S - 1) * a.ldx + a.v_off + (long long)grp * a.v_gs + 16 * mt + n];
           o[j] = p < a.S ? v : (__bf16)0.f;
         }
+        *reinterpret_cast<bf16x8*>(rec + ((PF_KTILES + mt) * 64 + lane) * 8) = o;
+      }
+    } else if (live) {
+      // 32 columns at a time: rows in 16-byte pieces (operand order, position blk_pos(n, c)), regrouped into the two
+      // 16-column tiles by products with an identity tile, which are exact (a non-finite value spreads over them, as it does
+      // over the head in the product with u_v). Element loads and the table in 4-byte loads took 5 us longer (three prompts of
+      // 200 42 -> 37 us in all, four of 512 71 -> 67).
+      bf16x8 id[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) id[h][j] = (8 * g + j == 16 * h + n) ? (__bf16)1.0f : (__bf16)0.0f;
+      const __bf16* xr[2];
+      bool in[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int p = 32 * jb + blk_pos(n, c);
+        in[c] = p < a.S;
+        xr[c] = xu + (long long)min(p, a.S - 1) * a.ldx + a.v_off + (long long)grp * a.v_gs;
+      }
+      bf16x8 x[4][2];                     // r_v <= 128 here
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int col = 32 * vb + 8 * g;
+          x[vb][c] = *reinterpret_cast<const bf16x8*>(xr[c] + (col < a.r_v ? col : 0));
+          if (!in[c]) x[vb][c] = bf16x8{};
+        }
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        if (16 * mt >= a.r_v) continue;
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        const bf16x8 o = pack8(mfma16(x[mt >> 1][0], id[mt & 1], z), mfma16(x[mt >> 1][1], id[mt & 1], z));
         *reinterpret_cast<bf16x8*>(rec + ((PF_KTILES + mt) * 64 + lane) * 8) = o;
       }
     }
@@ -212,7 +257,7 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
         float q[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) q[i] = acc[c][t][i];
-        rope_meta<4>(q, a.cos_t, a.sin_t, pr, 16 * t + 4 * g);
+        rope4(q, a.cos_t, a.sin_t, pr, 16 * t + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           acc[c][t][i] = q[i];
@@ -260,8 +305,13 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
 // Flash attention over the records. A workgroup owns PF_ROWS rows of one (user, KV head), a row being one
 // (position, query head of the group) in position-major order, so the group's heads share every K and V tile. A
 // wave owns NG column groups of 16 rows; its rotated, scaled query sits in registers as two planes. Each 32-key
-// record is copied to LDS once per workgroup (double buffered: the next one's loads are in flight during the
-// arithmetic) and every K tile read from LDS feeds up to 3 NG MFMAs. Scores are computed transposed
+// record is copied to LDS once per workgroup (three buffers, one barrier a record: record j + 2 is loaded during record j
+// and written at its end, so that the first K tiles of j + 1 can be read before the barrier) and every K tile read from LDS
+// feeds up to 2 NG MFMAs. K tiles are read one dim block ahead of their products and V tiles ahead of the softmax (two
+// buffers and reads where the compiler put them: 4096 positions at r 64 / 64 312 -> 309 us with the rebuild, 2048 at 64 /
+// 128 183 -> 172). Running half of the waves half a record behind the others, so that one half's softmax meets the other's
+// products, was slower (323 us). At 4096 positions the matrix cores are busy 44 % and the vector ALU 35 % of the time: a
+// softmax of eight keys costs a lane about 100 instructions beside 36 MFMAs. Scores are computed transposed
 // (keys x rows), so a lane holds eight keys of one row per column group: softmax in the exp2 domain with a lazily
 // refreshed maximum (cross-lane work only when a score passes it by 2^8), probabilities split into planes in
 // place, and they are the PV product's operand as they stand.
@@ -304,7 +354,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
         float t[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) t[i] = (float)xv[i];
-        rope_meta<4>(t, a.cos_t, a.sin_t, pr, d);
+        rope4(t, a.cos_t, a.sin_t, pr, d);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           v[kb][4 * hh + i] = t[i] * a.qscale;
@@ -329,7 +379,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
   auto put = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < LPW; ++i)
-      if (w + i * NW < NT) lds[(buf * NT + w + i * NW) * 64 + lane] = st[i];
+      lds[(buf * NT + min(w + i * NW, NT - 1)) * 64 + lane] = st[i];   // past the last tile: that one again, the same bytes
   };
 
   f32x4 O[NG][VT];
@@ -342,32 +392,70 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
     for (int t = 0; t < VT; ++t) O[gr][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
+  // Workgroup barrier over LDS: this wave's LDS writes and reads are done, its global loads stay in flight.
+  auto barrier = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
   load(0);
   put(0);
-  __syncthreads();
+  load(min(1, nst - 1));
+  put(1);
+  barrier();
+  // One dim block's K tiles (both planes and half-blocks), read a block ahead of their products; the scheduling fences
+  // keep the compiler from sinking each read to its use.
+  f16x8 kt2[2][2][2];
+  auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+  auto read_k = [&](f16x8 (&x)[2][2], const bf16x8* kt, int kb) {
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) x[pl][c] = __builtin_bit_cast(f16x8, kt[(8 * pl + c * 4 + kb) * 64]);
+  };
+  // The record's scale by a vector load a record ahead (a scalar load would make the LDS waits wait for it as well).
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  const float* kscale = a.ksc + (long long)uk * a.nblk + zero;
+  float ksc_next = kscale[0];
+  int buf = 0;
+  read_k(kt2[0], lds + lane, 0);
   for (int j = 0; j < nst; ++j) {
-    load(min(j + 1, nst - 1));
     const int base = j * BLK;
-    if (base <= w_hi) {                                     // uniform per wave
-      const bf16x8* kt = lds + (j & 1) * NT * 64 + lane;
-      const float ksc = load_uniform_f(a.ksc, (long long)uk * a.nblk + j);
-      f32x4 s[NG][2];
+    const bool live = base <= w_hi;       // uniform per wave
+    const bf16x8* kt = lds + buf * NT * 64 + lane;
+    const float ksc = ksc_next;
+    ksc_next = kscale[min(j + 1, nst - 1)];
+    load(min(j + 2, nst - 1));
+    fence();
+    f32x4 s[NG][2];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+    for (int gr = 0; gr < NG; ++gr)
 #pragma unroll
-        for (int gr = 0; gr < NG; ++gr) s[gr][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < 2; ++c) s[gr][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (live) {
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-          const f16x8 kh = __builtin_bit_cast(f16x8, kt[(c * 4 + kb) * 64]);
-          const f16x8 km = __builtin_bit_cast(f16x8, kt[(8 + c * 4 + kb) * 64]);
+      for (int kb = 0; kb < 4; ++kb) {
+        if (kb < 3) read_k(kt2[(kb + 1) & 1], kt, kb + 1);
+        fence();
+        // km qh + kh qm + kh qh
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(km, q[0][gr][kb], s[gr][c]);
+        for (int t = 0; t < 3; ++t)
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(kh, q[1][gr][kb], s[gr][c]);
+          for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(kh, q[0][gr][kb], s[gr][c]);
-        }
+            for (int gr = 0; gr < NG; ++gr) s[gr][c] = mfma16(kt2[kb & 1][t == 0][c], q[t == 1][gr][kb], s[gr][c]);
+        fence();
       }
+    }
+    const bf16x8* vt = kt + PF_KTILES * 64;
+    bf16x8 vh[VSPLIT ? 1 : VT];
+    if constexpr (!VSPLIT) {              // the V tiles, in flight during the softmax
+#pragma unroll
+      for (int t = 0; t < VT; ++t) vh[t] = vt[t * 64];
+      fence();
+    }
+    if (live) {
       if (base + BLK - 1 > w_lo) {                          // the diagonal: keys past a row's own position
 #pragma unroll
         for (int gr = 0; gr < NG; ++gr)
@@ -408,32 +496,55 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
         l_run[gr] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         split3x8(p, ph[gr], pm[gr], pl[gr]);
       }
-      const bf16x8* vt = kt + PF_KTILES * 64;
+      fence();
+      if constexpr (VSPLIT) {
+        // two V tiles (three planes each) at a time, read a pair ahead
+        static_assert(VT % 2 == 0, "V tiles are taken in pairs");
+        bf16x8 vv[2][3][2];
+        auto read_v = [&](bf16x8 (&x)[3][2], int t0) {
 #pragma unroll
-      for (int t = 0; t < VT; ++t) {
-        const bf16x8 vh = vt[t * 64];
-        if constexpr (VSPLIT) {
-          const bf16x8 vm = vt[(VT + t) * 64], vl = vt[(2 * VT + t) * 64];
+          for (int pl = 0; pl < 3; ++pl)
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vl, ph[gr], O[gr][t]);
+            for (int t = 0; t < 2; ++t) x[pl][t] = vt[(pl * VT + t0 + t) * 64];
+        };
+        read_v(vv[0], 0);
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vh, pl[gr], O[gr][t]);
+        for (int t0 = 0; t0 < VT; t0 += 2) {
+          const int cur = (t0 >> 1) & 1;
+          if (t0 + 2 < VT) read_v(vv[cur ^ 1], t0 + 2);
+          fence();
+          auto pv = [&](int pl, const bf16x8 (&pp)[NG]) {
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vm, pm[gr], O[gr][t]);
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vm, ph[gr], O[gr][t]);
-        } else {
-#pragma unroll
-          for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vh, pl[gr], O[gr][t]);
+              for (int gr = 0; gr < NG; ++gr) O[gr][t0 + t] = mfma16(vv[cur][pl][t], pp[gr], O[gr][t0 + t]);
+          };
+          pv(2, ph);
+          pv(0, pl);
+          pv(1, pm);
+          pv(1, ph);
+          pv(0, pm);
+          pv(0, ph);
+          fence();
         }
+      } else {
+        // one plane of P over all V tiles before the next: consecutive products have different accumulators
+        auto pv = [&](const bf16x8 (&pp)[NG]) {
 #pragma unroll
-        for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vh, pm[gr], O[gr][t]);
+          for (int t = 0; t < VT; ++t)
 #pragma unroll
-        for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vh, ph[gr], O[gr][t]);
+            for (int gr = 0; gr < NG; ++gr) O[gr][t] = mfma16(vh[t], pp[gr], O[gr][t]);
+        };
+        pv(pl);
+        pv(pm);
+        pv(ph);
       }
     }
-    put((j + 1) & 1);
-    __syncthreads();
+    fence();
+    buf = buf == 2 ? 0 : buf + 1;
+    put(buf == 2 ? 0 : buf + 1);
+    read_k(kt2[0], lds + buf * NT * 64 + lane, 0);   // the next record's first tiles: written a record ago
+    barrier();
   }
 
 #pragma unroll
@@ -491,7 +602,7 @@ template <int VT, bool VSPLIT, bool UP>
 int launch_attn(const PrefillArgs& a, hipStream_t s) {
   constexpr int NW = 8, NG = 2;
   auto kern = palu_prefill_attn_kernel<VT, VSPLIT, UP, NW, NG>;
-  constexpr int lds = 2 * (PF_KTILES + (VSPLIT ? 3 * VT : VT)) * 1024;
+  constexpr int lds = 3 * (PF_KTILES + (VSPLIT ? 3 * VT : VT)) * 1024;
   static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
