@@ -108,7 +108,7 @@ class PaluAttention(torch.nn.Module):
         wk = gw(state_dict[f"{P}.wk_lat_pad"], self.k_width)
         wv = gw(state_dict[f"{P}.wv_lat_pad"], self.r_v)
         # [nh hd + n_groups (k_width + r_v), dim]: held in the decode projection's tiled order
-        # (decoder_ops.DecodeLinear); the prefill multiplies by its nn.Linear-layout copy
+        # (decoder_ops.DecodeLinear), which the prefill multiplies by as well
         self.wqkv = decoder_ops.DecodeLinear(torch.cat([wq, wk, wv], dim=0).to(dev, bf).contiguous(),
                                              self.max_batch_size, single_slice=True)
         self.wo = state_dict[f"{ln}.wo.weight"].to(dev, bf).contiguous()

@@ -61,8 +61,7 @@ class Transformer(torch.nn.Module):
         t = lambda k: state_dict.pop(k).to(dev, bf)
         self.tok_embeddings = t("tok_embeddings.weight")
         self.norm_w = t("norm.weight")
-        # projections of the decode step, held in its tiled order (decoder_ops.DecodeLinear); the prefill
-        # multiplies by nn.Linear-layout copies made per call
+        # projections held in the decode step's tiled order (decoder_ops.DecodeLinear), for the prefill as well
         rows = args.max_batch_size
         self.output = decoder_ops.DecodeLinear(t("output.weight"), rows)         # [vocab, dim]
         self.layers = []
