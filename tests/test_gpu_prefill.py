@@ -84,7 +84,7 @@ def test_prefill_attention_wide_range(gpu):
     assert bool(torch.isfinite(out).all()) and ((out - exp).abs() / bound).max().item() <= 1.0
 
 
-@pytest.mark.parametrize("kf,qf,spike", [(0.0, 1.0, 1.0), (1e-25, 1e22, 1.0), (1e-12, 1e12, 1.0), (1.0, 1.0, 4096.0)])
+@pytest.mark.parametrize("kf,qf,spike", [(0.0, 1.0, 1.0), (1e-25, 1e25, 1.0), (1e-12, 1e12, 1.0), (1.0, 1.0, 4096.0)])
 def test_prefill_attention_plane_scales(gpu, kf, qf, spike):
     """The power-of-two scales of the score planes: keys that are all zero, keys and queries far apart in magnitude, and
     records whose keys differ by 2^12 (position 40's latent large, its products with the query kept small by it)."""

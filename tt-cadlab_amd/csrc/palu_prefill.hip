@@ -85,9 +85,9 @@ __device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8& h, bf16x8&
 // x = s (h + m) with fp16 planes h, m of x / s: s a power of two that puts the largest magnitude of the set that x belongs
 // to (amax) in [2^14, 2^15), so that no value saturates and the planes hold 22 bits of every value above amax 2^-17 (and an
 // absolute 2^-39 amax of the rest). A zero or non-finite amax gives s = 2^-15 (non-finite values stay so); s is at least
-// 2^-63, so that a product of two scales is a normal number.
+// 2^-115 (its reciprocal a normal number).
 __device__ __forceinline__ float plane_scale(float amax, float& inv) {
-  const int e = max(-48, min(126, __builtin_amdgcn_frexp_expf(amax))) - 15;
+  const int e = max(-100, min(126, __builtin_amdgcn_frexp_expf(amax))) - 15;
   inv = __builtin_amdgcn_ldexpf(1.f, -e);
   return __builtin_amdgcn_ldexpf(1.f, e);
 }
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
       bool up = false;
 #pragma unroll
       for (int gr = 0; gr < NG; ++gr) {
-        f[gr] = qsc[gr] * ksc;
+        f[gr] = fmaxf(qsc[gr] * ksc, 0x1p-126f);            // not 0: a masked score times it stays -inf
         bm[gr] = max8(s[gr][0], s[gr][1]) * f[gr];
         up = up || bm[gr] > m_run[gr] + LAZY_RESCALE_LOG2;
       }
