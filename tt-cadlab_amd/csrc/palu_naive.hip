@@ -25,7 +25,7 @@ struct RebuildArgs {
 // consecutive width-indices of the K tile (eight-byte stores, 512 contiguous bytes per instruction).
 // Bound by memory and latency: the latents in, 256 bytes per key and head out (from L2 again for the flash-decode), and
 // the fp32 table rows, once per head (from L2). Four rows of 2000 positions at r 64 / 64: rebuild 16 us, flash-decode
-// 13.5, a layer's step 56 us against 120 with the chain of torch launches before (tiles to rows, copies, GEMM, rotation).
+// 13.5, a layer's step 43 us against 120 with the chain of torch launches before (tiles to rows, copies, GEMM, rotation).
 // Loading a block's table rows ahead of its products took 22 us (the last block's loads of a next one are lost).
 template <bool TILED, int R>
 __global__ __launch_bounds__(256) void palu_rebuild_kernel(const RebuildArgs a) {

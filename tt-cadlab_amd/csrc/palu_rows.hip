@@ -13,7 +13,7 @@
 //
 // Bound: MFMA from some 500 rows on, the weight stream below. Measured (MI355X, weights rotated past the caches; the
 // library GEMM on an nn.Linear-layout copy, without the time to make the copy, in brackets): 2048 x 28672 x 4096
-// with SwiGLU 437 us = 1.10 PFLOP/s (391), 2048 x 4096 x 14336 226 us (222), 512 x 28672 x 4096 134 (104), 128 x 28672 x
+// with SwiGLU 427 us = 1.13 PFLOP/s (391), 2048 x 4096 x 14336 220 us (222), 512 x 28672 x 4096 134 (104), 128 x 28672 x
 // 4096 59.5 (57.1), 300 x 4096 x 14336 66 (74), 100 x 4096 x 14336 33.5 (49.4). First forms: activations through registers
 // (one stage ahead) 535 us at the first shape; 256-row workgroups with one wave per SIMD 653 to 740 us (the 256
 // accumulators and the stages do not fit without copies); waits left to the compiler 543 us.
