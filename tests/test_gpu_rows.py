@@ -50,3 +50,22 @@ def test_linear_rows_swiglu(gpu, m, f, k, rtw):
     bound = _half_step(exp) * 1.001 + 1.1 * eps * (xd.abs() @ gd.abs().T) * uv.abs() + eps * gv.abs() * (xd.abs() @ ud.abs().T) \
         + 2.0 ** -20 * exp.abs()
     assert ((y - exp).abs() / bound).max().item() <= 1.0
+
+
+def test_few_rows_on_two_streams(gpu):
+    """A prefill's products of at most 64 rows over one split weight, on two streams at once: each equals its result
+    alone bit for bit (the split partials belong to the call, not to the weight)."""
+    g = torch.Generator().manual_seed(3)
+    lin = ops.DecodeLinear((torch.randn(512, 8192, generator=g) * 0.05).to(torch.bfloat16).cuda(), 64)
+    assert lin.ks > 1, "the plan must split for this test"
+    xs = [torch.randn(m, 8192, generator=g).to(torch.bfloat16).cuda() for m in (37, 60)]
+    alone = [lin.rows(x).clone() for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    outs = [[], []]
+    for _ in range(40):
+        for s, x, o in zip(streams, xs, outs):
+            with torch.cuda.stream(s):
+                o.append(lin.rows(x))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, a) for a, o in zip(alone, outs) for y in o)

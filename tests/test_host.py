@@ -510,3 +510,17 @@ def test_tile_weight_layout_and_inverse():
         decoder_ops.tile_weight(torch.zeros(40, 64), 1)
     with pytest.raises(RuntimeError, match="rtw"):
         decoder_ops.tile_weight(torch.zeros(32, 64), 9)
+
+
+def test_prefill_rows_keep_off_the_decode_workspace(monkeypatch):
+    """DecodeLinear.rows (a prefill's product) must not write its split partials into the module's own workspace: the
+    decode step and its captured graph use that one, and prefills of other users, perhaps on other streams."""
+    from palu_tt import decoder_ops
+    lin = object.__new__(decoder_ops.DecodeLinear)
+    lin.tiled, lin.gate_up, lin.rtw, lin.ks = True, False, 1, 8
+    lin.weight, lin.workspace = torch.zeros(64, 2048), torch.zeros(1 << 20, dtype=torch.uint8)
+    seen = []
+    monkeypatch.setattr(decoder_ops, "linear_tiled",
+                        lambda x, w, rtw, ks, out=None, workspace=None, **kw: seen.append((ks, workspace)) or x)
+    lin.rows(torch.zeros(20, 2048))
+    assert seen == [(8, None)]

@@ -632,11 +632,12 @@ class DecodeLinear:
 
     def rows(self, x: torch.Tensor) -> torch.Tensor:
         """The projection of a prefill's rows [rows, k] (any number) as bf16 rows: x @ w.T, or silu(gate) * up of a pair.
-        A tiled weight is multiplied as it is held, up to 64 rows by the decode step's kernel."""
+        A tiled weight is multiplied as it is held, up to 64 rows by the decode step's kernel. Split partials go to memory
+        of this call: self.workspace is the decode step's, and a prefill may run beside it or another prefill."""
         if not self.tiled:
             return self(x)
         if not self.gate_up and x.shape[0] <= 64:
-            return self(x)
+            return linear_tiled(x, self.weight, self.rtw, self.ks)
         return linear_rows(x, self.weight, self.rtw, swiglu=self.gate_up)
 
     def plain(self) -> torch.Tensor:
