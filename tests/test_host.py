@@ -380,6 +380,29 @@ def test_flash_decode_and_append_envelope_errors(lib):
     assert rc == _native.PALU_EINVAL and "1..32 groups" in lib.palu_last_error().decode()
 
 
+@pytest.mark.parametrize("layout,r_v", [(1, 0), (1, -64), (1, 16), (1, 40), (1, 144), (0, 0), (0, 48)])
+def test_naive_decode_refuses_v_widths_before_any_launch(lib, layout, r_v):
+    """An r_v without a flash-decode kernel is refused as an argument, with the 16-byte workspace that the size query's
+    0 suggests: past the checks the rebuild would write its keys over whatever follows it."""
+    need = lib.palu_naive_workspace_bytes(2, 2, 64, r_v)
+    rc = lib.palu_naive_decode(_FAKE, _FAKE, _FAKE, _FAKE, _FAKE, 64, _FAKE, _FAKE, _FAKE, 0.1, 2, 8, 2, 64, 64, 64, r_v, 1,
+                               layout, 0, _FAKE, max(need, 16), None)
+    assert rc == _native.PALU_EUNSUPPORTED and "r_v" in lib.palu_last_error().decode()
+
+
+def test_naive_decode_envelope_errors(lib):
+    def call(batch=2, n_q=8, n_kv=2, ws=1 << 30):
+        rc = lib.palu_naive_decode(_FAKE, _FAKE, _FAKE, _FAKE, _FAKE, 64, _FAKE, _FAKE, _FAKE, 0.1, batch, n_q, n_kv, 64, 64,
+                                   64, 64, 1, 1, 0, _FAKE, ws, None)
+        return rc, lib.palu_last_error().decode()
+    for kw, code, needle in (({"batch": 0}, _native.PALU_EINVAL, "positive"), ({"n_kv": -2}, _native.PALU_EINVAL, "positive"),
+                             ({"batch": 40000}, _native.PALU_EUNSUPPORTED, "grid limit"),
+                             ({"n_q": 7}, _native.PALU_EINVAL, "KV head count"),
+                             ({"ws": lib.palu_naive_workspace_bytes(2, 2, 64, 64) - 1}, _native.PALU_EINVAL, "workspace")):
+        rc, msg = call(**kw)
+        assert rc == code and needle in msg, (kw, rc, msg)
+
+
 def test_fused_projection_plans_and_envelope_errors(lib):
     """The one-slice plan the fused epilogues use, and their argument checks (host-side, before any launch)."""
     rtw, ks = ctypes.c_int(0), ctypes.c_int(0)

@@ -170,6 +170,11 @@ extern "C" int palu_naive_decode(const void* q, const void* k_latent, const void
     return fail(PALU_EINVAL, "%s: recon_len %d of a cache of %d positions (multiples of 32 when tiled)", who, recon_len, seq_len);
   if (r_k <= 0 || r_k > HD || r_k % (tiled ? 16 : 32))
     return fail(PALU_EINVAL, "%s: r_k %d (multiples of 32 up to %d; of 16 for tiled caches)", who, r_k, HD);
+  if (batch <= 0 || n_kv <= 0) return fail(PALU_EINVAL, "%s: batch and head counts must be positive", who);
+  if ((long long)batch * n_kv > 65535) return fail(PALU_EUNSUPPORTED, "%s: batch * n_kv exceeds the grid limit", who);
+  // The flash-decode's V widths, checked ahead of the rebuild's launch: the workspace's size depends on a valid one.
+  if (r_v < 32 || r_v > HD || r_v % (tiled ? 16 : 32))
+    return fail(PALU_EUNSUPPORTED, "%s: r_v %d (multiples of 32 up to %d; of 16 from 32 on for tiled caches)", who, r_v, HD);
   if (table_rows < recon_len) return fail(PALU_EINVAL, "%s: %d table rows for %d positions", who, table_rows, recon_len);
   if (!al16(u_k) || !al16(cos_table) || !al16(sin_table) || !al16(workspace))
     return fail(PALU_EINVAL, "%s: 16-byte alignment required", who);
@@ -177,7 +182,7 @@ extern "C" int palu_naive_decode(const void* q, const void* k_latent, const void
   if (workspace_bytes < need)
     return fail(PALU_EINVAL, "%s: workspace of %zu bytes needed (palu_naive_workspace_bytes), got %zu", who, need, workspace_bytes);
   DecodeArgs a;
-  const size_t kb = key_bytes(batch > 0 ? batch : 0, n_kv > 0 ? n_kv : 0, recon_len);
+  const size_t kb = key_bytes(batch, n_kv, recon_len);
   if (int rc = palu::flash_setup(a, q, workspace, v_latent, cur_pos, out, scale, batch, n_q, n_kv, recon_len, r_v, out_dtype,
                                  cache_layout, deterministic, static_cast<char*>(workspace) + kb, workspace_bytes - kb, who))
     return rc;
