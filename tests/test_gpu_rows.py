@@ -37,6 +37,14 @@ def test_linear_rows(gpu, m, n, k, rtw):
     assert ((y - exp).abs() / bound).max().item() <= 1.0
 
 
+# one row block of two-tile waves (n at most 64 workgroups' columns) and of four-tile waves, with 0 to 3 stages past the
+# last whole round of four, odd slices among them: the last stages wait for copies that the main loop's counts don't cover
+@pytest.mark.parametrize("k32", [6, 7, 14, 15, 22, 24, 30, 31, 60, 62])
+@pytest.mark.parametrize("m,n", [(128, 1024), (96, 512), (300, 16384)])
+def test_linear_rows_last_stages(gpu, m, n, k32):
+    test_linear_rows(gpu, m, n, 32 * k32, 2)
+
+
 @pytest.mark.parametrize("m,f,k,rtw", [(65, 32, 32, 1), (130, 96, 224, 7), (257, 544, 96, 3), (128, 1024, 512, 4), (33, 64, 64, 8)])
 def test_linear_rows_swiglu(gpu, m, f, k, rtw):
     x, g = _case(m, f, k, f + k)

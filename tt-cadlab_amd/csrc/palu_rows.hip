@@ -104,7 +104,8 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
                                        (lvoid*)(buf + ((i & 1) * MT + w * (XPW / 2) + (i >> 1)) * 64), 16, 0, 0);
     }
   };
-  auto stage = [&](const bf16x8* cur, bf16x8* nxt, int j, int s) __attribute__((always_inline)) {
+  // `tail`: one of the last nst % 4 stages (a constant where it is called), whose copies ahead would be past the slice.
+  auto stage = [&](const bf16x8* cur, bf16x8* nxt, int j, int s, bool tail) __attribute__((always_inline)) {
     // The stage's activation tiles in pairs, each pair read from LDS while the one before it is multiplied (left to the
     // compiler every read stood right before its use), and the products ahead of the other workgroup's address work: 2048 x
     // 28672 x 4096 434 -> 427 us, 2048 x 4096 x 14336 223 -> 220.
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
       for (int i = 0; i < 2; ++i) b[q & 1][i] = cur[(2 * q + i) * 64 + lane];
     };
     read(0);
-    load_x(nxt, s + XS - 1);
+    if (!tail) load_x(nxt, s + XS - 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < MT; ++q) {        // k tile q / (MT / 2), row tiles 2 q % MT and the next
@@ -133,11 +134,14 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
     }
     // Loads complete in order. The next stage's activations were asked for XS - 2 stages ago and its weights WS - 1
     // stages ago, so once no more than the loads of that many stages are outstanding, both have arrived, and past the
-    // barrier in every wave. (Left to the compiler the weights' wait was for every load.)
+    // barrier in every wave. (Left to the compiler the weights' wait was for every load.) That count holds where every
+    // stage issues all its loads; a tail stage does not (it copies nothing, and the compiler drops weight loads that no
+    // stage uses), so it waits for everything.
     __builtin_amdgcn_sched_barrier(0);
     constexpr int V = (WS - 1 < XS - 2 ? WS - 1 : XS - 2) * (XPW + 2 * RPW);
     static_assert(V < 64, "the wait counter");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (V & 15) | ((V >> 4) << 14));
+    if (tail) __builtin_amdgcn_s_waitcnt(0x0F70);
+    else __builtin_amdgcn_s_waitcnt(0x0F70 | (V & 15) | ((V >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -156,14 +160,14 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     int s = 0;
     for (; s + 4 <= nst; s += 4) {
-      stage(xs0, xs3, 0, s);
-      stage(xs1, xs0, 1, s + 1);
-      stage(xs2, xs1, 2, s + 2);
-      stage(xs3, xs2, 3, s + 3);
+      stage(xs0, xs3, 0, s, false);
+      stage(xs1, xs0, 1, s + 1, false);
+      stage(xs2, xs1, 2, s + 2, false);
+      stage(xs3, xs2, 3, s + 3, false);
     }
-    if (s < nst) stage(xs0, xs3, 0, s);
-    if (s + 1 < nst) stage(xs1, xs0, 1, s + 1);
-    if (s + 2 < nst) stage(xs2, xs1, 2, s + 2);
+    if (s < nst) stage(xs0, xs3, 0, s, true);
+    if (s + 1 < nst) stage(xs1, xs0, 1, s + 1, true);
+    if (s + 2 < nst) stage(xs2, xs1, 2, s + 2, true);
   }
   if (kt_n & 1) {                         // an odd slice's last k tile, straight from memory
     const int kt = kt_n - 1;
