@@ -403,8 +403,10 @@ int palu_latent_fill(void* cache, long long batch_stride, long long group_stride
  * [users * seq][ld]: query heads at columns 0 .. n_heads * 128 - 1, group g's K latent at k_col_offset + g * r_k and V
  * latent at v_col_offset + g * r_v. out[u * seq + p][h * 128 ..] (bf16, rows ld_out apart) = softmax(q K^T scale) V over
  * positions 0 .. p with K = RoPE(lat u_k), V = lat u_v (u_k / u_v [n_kv][r][128]; NULL with one 128-wide group per KV
- * head: the columns are K / V themselves). Keys, values, scores, probabilities and sums have fp32 precision; the
- * result is rounded to bf16 once. Ranks are multiples of 16. workspace: palu_prefill_workspace_bytes, 16-byte aligned. */
+ * head: the columns are K / V themselves). Keys and values are rebuilt, and all sums kept, in fp32. For the score products
+ * a rotated key and a scaled query are each taken as two fp16 planes over a power of two of their own: 22 bits of every
+ * element within 2^17 of the vector's largest, an absolute 2^-39 of that below. Probabilities and rebuilt values enter
+ * their products with 24 bits. The result is rounded to bf16 once. Ranks are multiples of 16. workspace: palu_prefill_workspace_bytes, 16-byte aligned. */
 int palu_prefill_attention(const void* qkv, long long ld, int users, int seq, int n_heads, int n_kv, int n_groups,
                            int k_col_offset, int r_k, const void* u_k, int v_col_offset, int r_v, const void* u_v,
                            const float* cos_table, const float* sin_table, int table_rows, float scale, void* out,

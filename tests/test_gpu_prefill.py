@@ -100,6 +100,24 @@ def test_prefill_attention_plane_scales(gpu, kf, qf, spike):
     assert ((out - exp).abs() / bound).max().item() <= 1.0
 
 
+@pytest.mark.parametrize("nkv,G,rv", [(2, 2, 64), (4, 2, 96)])
+@pytest.mark.parametrize("spike", [2.0 ** 20, 2.0 ** 28, float("inf"), float("-inf")])
+def test_prefill_attention_one_key_out_of_line(gpu, nkv, G, rv, spike):
+    """One key far above the others of its 32 (or infinite): the rows before it, which don't see it, keep their results bit
+    for bit, and the rows after it stay at the bound of test_prefill_attention where its score is that of one key among
+    others or rules it out (its products with these queries are above 1e3 in size)."""
+    x, k0, v0, u_k, u_v, cos, sin = _inputs(1, 96, 8, nkv, G, 64, rv, 9)
+    run = lambda t: decoder_ops.prefill_attention(t, 1, 8, nkv, G, k0, 64, u_k, v0, rv, u_v, cos, sin, HD ** -0.5)
+    y = x.clone()
+    y[40, k0:v0] *= spike
+    out = run(y)
+    assert torch.equal(out[:40], run(x)[:40])
+    if abs(spike) != float("inf"):
+        exp = _exact(y, 1, 8, nkv, G, k0, 64, u_k, v0, rv, u_v, cos, sin, HD ** -0.5)
+        bound = _half_step(exp) * 1.001 + 4e-6 * exp.abs().amax(-1, keepdim=True)
+        assert ((out.double() - exp).abs() / bound).max().item() <= 1.0
+
+
 def test_prefill_whole_v_heads_keep_a_nonfinite_value_in_its_column(gpu):
     x, k0, v0, u_k, _, cos, sin = _inputs(1, 64, 4, 1, 1, 64, HD, 3, full_v=True)
     x = x.clone()

@@ -9,8 +9,8 @@
 //   3. palu_prefill_attn_kernel: flash attention.
 //
 // Precision on 16-bit matrix cores. Scores: q and K are each the sum of two fp16 planes of their value over a power-of-two
-// scale (plane_scale: one per query row and one per 32-key record, applied again in the exponent), 22 bits, and a
-// product is three MFMAs, hm + mh + hh. Probabilities (and a rebuilt V) are the sum of three bf16 planes h + m + l (24
+// scale (plane_scale: one per query row and one per key, applied again to the scores), 22 bits, and a product is
+// three MFMAs, hm + mh + hh. Probabilities (and a rebuilt V) are the sum of three bf16 planes h + m + l (24
 // bits, and bf16 has fp32's range); with a V latent, which is exactly bf16, a product is three MFMAs, between two such
 // sums six (terms below 2^-24 dropped). All sums are fp32. Measured against 64 bits over 17 to 4096 positions, ranks 32 to
 // 512 and scores of spread 1 and 4, the result before its bf16 rounding is off by 2.3e-7 to 1.06e-6 (relative 2-norm);
@@ -44,7 +44,7 @@ struct PrefillArgs {
   int table_rows;
   float qscale;                           // softmax scale * log2 e
   __bf16* rec;                            // records [U * nkv][nblk][tiles][64][8] (K tiles fp16, V tiles bf16)
-  float* ksc;                             // power-of-two scale of a record's K planes [U * nkv][nblk]
+  float* ksc;                             // power-of-two scales of the keys' planes [U * nkv][nblk][32]
   __bf16* uvt;                            // u_v^T tiles [nkv][KBV][8][64][8] (up-projection)
   __bf16* out;                            // [U * S][ldo]
   long long ldo;
@@ -82,15 +82,21 @@ __device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8& h, bf16x8&
   }
 }
 
-// x = s (h + m) with fp16 planes h, m of x / s: s a power of two that puts the largest magnitude of the set that x belongs
-// to (amax) in [2^14, 2^15), so that no value saturates and the planes hold 22 bits of every value above amax 2^-17 (and an
-// absolute 2^-39 amax of the rest). A zero or non-finite amax gives s = 2^-15 (non-finite values stay so); s is at least
-// 2^-115 (its reciprocal a normal number).
+// x = s (h + m) with fp16 planes h, m of x / s: s a power of two that puts the largest magnitude of the key or query that
+// x belongs to (amax) in [2^14, 2^15), so that the planes hold 22 bits of every value above amax 2^-17 (and an
+// absolute 2^-39 amax of the rest). Each key has its own scale: with one for the 32 keys of a record (until then 16
+// multiplications a record and lane fewer: 4096 positions at r 64 / 64 323.8 us against 325.3, two prompts of 777 with
+// grouped latents 110.1, 111.3) a key 2^24 times the others left these 1e-3 of error in their scores, and an infinite
+// one made them NaN.
 __device__ __forceinline__ float plane_scale(float amax, float& inv) {
   const int e = max(-100, min(126, __builtin_amdgcn_frexp_expf(amax))) - 15;
   inv = __builtin_amdgcn_ldexpf(1.f, -e);
   return __builtin_amdgcn_ldexpf(1.f, e);
 }
+
+// A score is (sum of plane products) x key scale x row scale; between the two products it carries this power of two, which
+// keeps it and both factors in range for keys up to 2^118 and any query.
+constexpr float KEY_SCALE = 0x1p-14f;
 
 __device__ __forceinline__ void split2x8(const float (&v)[8], float inv, f16x8& h, f16x8& m) {
 #pragma unroll
@@ -248,10 +254,10 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
   if (!live) return;
   if (!isv) {
     // lane (n, g), tile c: dims 16 t + 4 g + i of position blk_pos(n, c); two tiles make one operand slot
-    float amax = 0.f;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int pr = min(p[c], a.table_rows - 1);
+      float amax = 0.f;
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         float q[4];
@@ -264,14 +270,9 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
           amax = fmaxf(amax, fabsf(q[i]));
         }
       }
-    }
-#pragma unroll
-    for (int o = 1; o < 64; o *= 2) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-    float inv;
-    const float sc = plane_scale(amax, inv);
-    if (lane == 0) a.ksc[(long long)uk * a.nblk + jb] = sc;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
+      float inv;
+      const float sc = plane_scale(wave_max_xor48(amax), inv);   // over the key's four lanes
+      if (g == 0) a.ksc[((long long)uk * a.nblk + jb) * BLK + blk_pos(n, c)] = sc * KEY_SCALE;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
         float v[8];
@@ -283,6 +284,7 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
         *reinterpret_cast<f16x8*>(o) = h;
         *reinterpret_cast<f16x8*>(o + 8 * 512) = m;
       }
+    }
   } else {
     // lane (n, g), tile t: column 16 t + n at positions 8 g + 4 c + i
     bf16x8 h, m, l;
@@ -362,7 +364,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
         }
       }
     float inv;
-    qsc[gr] = plane_scale(wave_max_xor48(amax), inv);       // over the row's four lanes
+    qsc[gr] = plane_scale(wave_max_xor48(amax), inv) / KEY_SCALE;   // over the row's four lanes
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) split2x8(v[kb], inv, q[0][gr][kb], q[1][gr][kb]);
   }
@@ -413,19 +415,15 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
 #pragma unroll
       for (int c = 0; c < 2; ++c) x[pl][c] = __builtin_bit_cast(f16x8, kt[(8 * pl + c * 4 + kb) * 64]);
   };
-  // The record's scale by a vector load a record ahead (a scalar load would make the LDS waits wait for it as well).
-  int zero = 0;
-  asm volatile("" : "+v"(zero));
-  const float* kscale = a.ksc + (long long)uk * a.nblk + zero;
-  float ksc_next = kscale[0];
+  // The scales of this lane's keys, loaded before the record's barrier.
+  const f32x4* kscale = reinterpret_cast<const f32x4*>(a.ksc + (long long)uk * a.nblk * BLK + 8 * g);
+  f32x4 ksc[2] = {kscale[0], kscale[1]};
   int buf = 0;
   read_k(kt2[0], lds + lane, 0);
   for (int j = 0; j < nst; ++j) {
     const int base = j * BLK;
     const bool live = base <= w_hi;       // uniform per wave
     const bf16x8* kt = lds + buf * NT * 64 + lane;
-    const float ksc = ksc_next;
-    ksc_next = kscale[min(j + 1, nst - 1)];
     load(min(j + 2, nst - 1));
     fence();
     f32x4 s[NG][2];
@@ -465,12 +463,15 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
             for (int i = 0; i < 4; ++i)
               if (base + 8 * g + 4 * c + i > pos[gr]) s[gr][c][i] = NEG_INF;
       }
-      float f[NG], bm[NG];                                  // the planes' scales go into the exponent
+      float bm[NG];                                         // the keys' scales here, the row's in the exponent
       bool up = false;
 #pragma unroll
       for (int gr = 0; gr < NG; ++gr) {
-        f[gr] = fmaxf(qsc[gr] * ksc, 0x1p-126f);            // not 0: a masked score times it stays -inf
-        bm[gr] = max8(s[gr][0], s[gr][1]) * f[gr];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[gr][c][i] *= ksc[c][i];
+        bm[gr] = max8(s[gr][0], s[gr][1]) * qsc[gr];
         up = up || bm[gr] > m_run[gr] + LAZY_RESCALE_LOG2;
       }
       if (__any(up)) {
@@ -492,7 +493,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) p[4 * c + i] = __builtin_amdgcn_exp2f(fmaf(s[gr][c][i], f[gr], -mref));
+          for (int i = 0; i < 4; ++i) p[4 * c + i] = __builtin_amdgcn_exp2f(fmaf(s[gr][c][i], qsc[gr], -mref));
         l_run[gr] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         split3x8(p, ph[gr], pm[gr], pl[gr]);
       }
@@ -543,6 +544,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void palu_prefill_attn_ke
     fence();
     buf = buf == 2 ? 0 : buf + 1;
     put(buf == 2 ? 0 : buf + 1);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) ksc[c] = kscale[min(j + 1, nst - 1) * (BLK / 4) + c];
     read_k(kt2[0], lds + buf * NT * 64 + lane, 0);   // the next record's first tiles: written a record ago
     barrier();
   }
@@ -690,7 +693,7 @@ bool prefill_shape_ok(int users, int seq, int n_heads, int n_kv, int n_groups, i
 extern "C" size_t palu_prefill_workspace_bytes(int users, int seq, int n_heads, int n_kv, int n_groups, int r_k, int r_v) {
   if (!prefill_shape_ok(users, seq, n_heads, n_kv, n_groups, r_k, r_v)) return 0;
   const size_t blocks = (size_t)users * n_kv * ((seq + 31) / 32);
-  return blocks * (PF_KTILES + v_tiles(n_kv, n_groups, r_v)) * 1024 + (size_t)n_kv * 4 * 8 * 1024 + blocks * sizeof(float);
+  return blocks * (PF_KTILES + v_tiles(n_kv, n_groups, r_v)) * 1024 + (size_t)n_kv * 4 * 8 * 1024 + blocks * BLK * sizeof(float);
 }
 
 extern "C" int palu_prefill_attention(const void* qkv, long long ld, int users, int seq, int n_heads, int n_kv, int n_groups,

@@ -181,8 +181,9 @@ def prefill_attention(qkv: torch.Tensor, users: int, n_heads: int, n_kv: int, n_
                       sin: torch.Tensor, scale: float) -> torch.Tensor:
     """Causal attention of `users` prompts from their QKV projection rows qkv [users * seq, ...] (bf16): query heads,
     then group g's K latent at column k_col + g * r_k and V latent at v_col + g * r_v; K = RoPE(lat @ u_k), V = lat @ u_v
-    (None: the columns are K / V heads themselves), in fp32 precision throughout. Returns bf16 [users * seq, n_heads *
-    128]."""
+    (None: the columns are K / V heads themselves). K, V and all sums are fp32; a key and a query enter the score products
+    as two fp16 planes over their own power of two (22 bits within 2^17 of the vector's largest element), probabilities
+    and V with 24 bits. Returns bf16 [users * seq, n_heads * 128]."""
     _check(qkv, "qkv")
     _check(cos, "cos", torch.float32)
     _check(sin, "sin", torch.float32)
