@@ -118,6 +118,25 @@ def test_prefill_attention_one_key_out_of_line(gpu, nkv, G, rv, spike):
         assert ((out.double() - exp).abs() / bound).max().item() <= 1.0
 
 
+@pytest.mark.parametrize("value", [3e38, -3e38, float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("full_k", [True, False])
+def test_prefill_attention_key_at_the_end_of_the_range(gpu, full_k, value):
+    """One element of one key (or of its latent) at the end of bf16's range or not finite: results are finite where the
+    64-bit ones are (rows before it, and those where its score is -inf), at the bound, and NaN where they are."""
+    rk = HD if full_k else 64
+    x, k0, v0, u_k, u_v, cos, sin = _inputs(1, 96, 8, 2, 2, rk, 64, 12, full_k=full_k)
+    x = x.clone()
+    x[40, [k0 + 6, k0 + rk + 9]] = value
+    out = decoder_ops.prefill_attention(x, 1, 8, 2, 2, k0, rk, u_k, v0, 64, u_v, cos, sin, HD ** -0.5).double()
+    exp = _exact(x, 1, 8, 2, 2, k0, rk, u_k, v0, 64, u_v, cos, sin, HD ** -0.5)
+    exp, out = exp.view(96, 8, HD), out.view(96, 8, HD)
+    fin = torch.isfinite(exp)
+    assert torch.equal(torch.isfinite(out), fin) and bool(fin[:40].all())
+    exp, out = exp.nan_to_num(0.0), out.nan_to_num(0.0)
+    bound = _half_step(exp) * 1.001 + 4e-6 * exp.abs().amax(-1, keepdim=True) + 1e-30
+    assert ((out - exp).abs() / bound).max().item() <= 1.0
+
+
 def test_prefill_whole_v_heads_keep_a_nonfinite_value_in_its_column(gpu):
     x, k0, v0, u_k, _, cos, sin = _inputs(1, 64, 4, 1, 1, 64, HD, 3, full_v=True)
     x = x.clone()

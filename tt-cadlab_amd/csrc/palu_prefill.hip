@@ -87,16 +87,17 @@ __device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8& h, bf16x8&
 // absolute 2^-39 amax of the rest). Each key has its own scale: with one for the 32 keys of a record (until then 16
 // multiplications a record and lane fewer: 4096 positions at r 64 / 64 323.8 us against 325.3, two prompts of 777 with
 // grouped latents 110.1, 111.3) a key 2^24 times the others left these 1e-3 of error in their scores, and an infinite
-// one made them NaN.
+// one made them NaN. amax is that of the finite values; 0 gives s = 2^-15.
 __device__ __forceinline__ float plane_scale(float amax, float& inv) {
-  const int e = max(-100, min(126, __builtin_amdgcn_frexp_expf(amax))) - 15;
+  const int e = max(-100, __builtin_amdgcn_frexp_expf(amax)) - 15;   // at most 128 - 15: inv is a normal number
   inv = __builtin_amdgcn_ldexpf(1.f, -e);
   return __builtin_amdgcn_ldexpf(1.f, e);
 }
 
 // A score is (sum of plane products) x key scale x row scale; between the two products it carries this power of two, which
-// keeps it and both factors in range for keys up to 2^118 and any query.
-constexpr float KEY_SCALE = 0x1p-14f;
+// keeps it and both factors in range: keys up to 2^122 in all 128 dims at once (2^127 in a few) and any bf16 query.
+constexpr float KEY_SCALE = 0x1p-18f;
+constexpr float INF = __builtin_inff();
 
 __device__ __forceinline__ void split2x8(const float (&v)[8], float inv, f16x8& h, f16x8& m) {
 #pragma unroll
@@ -270,8 +271,19 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
           amax = fmaxf(amax, fabsf(q[i]));
         }
       }
+      amax = wave_max_xor48(amax);                              // over the key's four lanes
+      const bool inf = amax == INF;
+      if (__any(inf)) {
+        float fin = 0.f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) fin = fmaxf(fin, fabsf(acc[c][t][i]) < INF ? fabsf(acc[c][t][i]) : 0.f);
+        fin = wave_max_xor48(fin);
+        amax = inf ? fin : amax;
+      }
       float inv;
-      const float sc = plane_scale(wave_max_xor48(amax), inv);   // over the key's four lanes
+      const float sc = plane_scale(amax, inv);
       if (g == 0) a.ksc[((long long)uk * a.nblk + jb) * BLK + blk_pos(n, c)] = sc * KEY_SCALE;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
@@ -280,6 +292,16 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
         for (int i = 0; i < 8; ++i) v[i] = acc[c][2 * kb + (i >> 2)][i & 3];
         f16x8 h, m;
         split2x8(v, inv, h, m);
+        if (inf) {
+          // An infinite value goes to the m plane alone, which meets only the query's h plane: its score is then
+          // infinite, or NaN where infinities of both signs meet, as the product in fp32 is.
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (fabsf(v[j]) == INF) {
+              h[j] = (_Float16)0.f;
+              m[j] = (_Float16)v[j];
+            }
+        }
         __bf16* o = rec + ((c * 4 + kb) * 64 + lane) * 8;
         *reinterpret_cast<f16x8*>(o) = h;
         *reinterpret_cast<f16x8*>(o + 8 * 512) = m;
