@@ -205,6 +205,15 @@ def test_layer_prefill_matches_the_torch_path(gpu, rk, rv, gs, layout, group_ran
             assert torch.equal(got[i], store)
 
 
+def test_layer_prefill_takes_unaligned_prompts(gpu):
+    """A prompt that starts off a 16-byte boundary (a view into a larger buffer) gives what an aligned copy gives."""
+    att, g = _layer(64, 64, 1, "tiled", 1, 64)
+    buf = torch.randn(1 + 20 * 256, generator=g).to(torch.bfloat16).cuda()
+    x = buf[1:].view(1, 20, 256)
+    assert x.data_ptr() % 16
+    assert torch.equal(att.forward(x, mode="prefill"), att.forward(x.clone(), mode="prefill"))
+
+
 def test_layer_prefill_keeps_autograd(gpu):
     att, g = _layer(64, 64, 1, "rows", 1, 64)
     x = torch.randn(1, 20, 256, generator=g).cuda().requires_grad_()

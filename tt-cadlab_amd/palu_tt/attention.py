@@ -297,7 +297,8 @@ class PaluAttention(torch.nn.Module):
         assert 0 < S <= self.max_seq_len and user_id + U <= self.max_batch_size
         if (U > 0 and user_id >= 0 and self.head_dim == 128 and decoder_ops.kernels_can_take(
                 x, self.wqkv.weight, self.wo, self.u_k, self.u_v, *(self._store(c) for c in self.layer_past))):
-            return self._prefill_kernels(x3.reshape(U * S, -1).contiguous(), U, user_id).reshape(*shape[:-1], self.hidden_size)
+            x2 = decoder_ops.aligned(x3.reshape(U * S, -1))
+            return self._prefill_kernels(x2, U, user_id).reshape(*shape[:-1], self.hidden_size)
         outs = []
         for u in range(U):
             outs.append(self._prefill_one(x3[u], user_id + u))

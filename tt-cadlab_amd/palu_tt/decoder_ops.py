@@ -20,6 +20,13 @@ def _check(t: torch.Tensor, name: str, dtype=torch.bfloat16) -> None:
         raise RuntimeError(f"{name} must be a {dtype} tensor on the GPU")
 
 
+def aligned(t: torch.Tensor) -> torch.Tensor:
+    """A contiguous tensor as the kernels read it, 16 bytes at a time: t, or a copy where it starts off a 16-byte boundary
+    (a view into another tensor)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, res: Optional[torch.Tensor] = None,
             h_out: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
             tiled_out: bool = False, res_part: Optional[torch.Tensor] = None) -> torch.Tensor:
