@@ -115,6 +115,37 @@ def test_decoder_above_64_rows_matches_lowrank_llama(gpu):
         _check(out, exp[:, S + t], f"decode step {t}")
 
 
+def _as_views(sd, keys):
+    """The named tensors as views with the same values: off a 16-byte boundary, or (vectors) with a stride of 2."""
+    for k in keys:
+        t = sd[k]
+        buf = torch.empty(2 * t.numel() + 1, dtype=t.dtype, device=t.device)
+        view = buf[1:1 + 2 * t.numel():2] if t.dim() == 1 else buf[1:1 + t.numel()].view(t.shape)
+        sd[k] = view.copy_(t)
+
+
+@pytest.mark.parametrize("use_fused_k", [True, False])
+def test_weights_as_views_of_larger_buffers(gpu, use_fused_k):
+    """A state dict on the GPU whose norm weights and factors are strided or unaligned views: prefill and (naive path)
+    decode give what the same model with contiguous ones gives."""
+    args = lambda: pm.ModelArgs(dim=256, n_layers=1, n_heads=4, n_kv_heads=2, vocab_size=320, ffn_dim=512, max_seq_len=64,
+                                max_batch_size=2)
+    logits = []
+    for views in (False, True):
+        a = args()
+        sd = pm.random_palu_state_dict(a, [64], [32], gpu, seed=5, std=0.05, use_fused_k=use_fused_k)
+        a.palu.runtime.deterministic = True
+        for k in ("norm.weight", "layers.0.attention_norm.weight", "layers.0.ffn_norm.weight"):
+            sd[k] = (1 + 0.3 * torch.randn(256, generator=torch.Generator().manual_seed(len(k)))).to(gpu, torch.bfloat16)
+        if views:
+            _as_views(sd, ["norm.weight", "layers.0.attention_norm.weight", "layers.0.ffn_norm.weight",
+                           "layers.0.attention.palu.u_k", "layers.0.attention.palu.u_v"])
+        net = pm.Transformer(a, sd, gpu)
+        ids = torch.arange(40, device=gpu).view(2, 20) * 7
+        logits.append((net.prefill(ids), net.decode(ids[:, 0], torch.full((2,), 20, dtype=torch.int32, device=gpu))))
+    assert torch.equal(logits[0][0], logits[1][0]) and torch.equal(logits[0][1], logits[1][1])
+
+
 def test_generate_greedy_is_consistent_with_decode(gpu):
     """generate() (graph decode) returns, at every step, the argmax of the eager decode's logits for the
     tokens it generated (teacher-forced replay on a fresh model built from the same seed)."""

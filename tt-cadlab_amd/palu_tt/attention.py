@@ -119,9 +119,10 @@ class PaluAttention(torch.nn.Module):
         self.wo_out = decoder_ops.DecodeLinear(wo_fused.view(-1, self.n_heads, self.head_dim)[:, :, :self.out_width]
                                                .reshape(-1, self.n_heads * self.out_width).contiguous(),
                                                self.max_batch_size, single_slice=True)
-        self.u_k = state_dict[f"{P}.u_k"].to(dev, bf).contiguous() if self.recon_k else None   # [nkv, r_k, hd]
+        factor = lambda k: decoder_ops.aligned(state_dict[f"{P}.{k}"].to(dev, bf))
+        self.u_k = factor("u_k") if self.recon_k else None                                      # [nkv, r_k, hd]
         self.w_rot = state_dict[f"{P}.w_rot"].to(dev, bf)[None].contiguous() if self.recon_k else None
-        self.u_v = state_dict[f"{P}.u_v"].to(dev, bf).contiguous() if self.recon_v else None   # [nkv, r_v, hd]
+        self.u_v = factor("u_v") if self.recon_v else None                                      # [nkv, r_v, hd]
 
         cos, sin = fused.cos_sin_tables(hd, self.max_seq_len, configuration.rope_theta,
                                         getattr(configuration, "rope_scaling", None))

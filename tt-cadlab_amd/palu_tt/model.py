@@ -60,7 +60,8 @@ class Transformer(torch.nn.Module):
         bf, dev = torch.bfloat16, self.device
         t = lambda k: state_dict.pop(k).to(dev, bf)
         self.tok_embeddings = t("tok_embeddings.weight")
-        self.norm_w = t("norm.weight")
+        norm = lambda k: decoder_ops.aligned(t(k))
+        self.norm_w = norm("norm.weight")
         # projections held in the decode step's tiled order (decoder_ops.DecodeLinear), for the prefill as well
         rows = args.max_batch_size
         self.output = decoder_ops.DecodeLinear(t("output.weight"), rows)         # [vocab, dim]
@@ -73,12 +74,12 @@ class Transformer(torch.nn.Module):
                 state_dict.pop(k)
             # the FFN norm's weight is folded into a tiled gate / up weight (then the norm in front of it
             # multiplies by ones, and the decode step normalises inside the gate / up launch)
-            ffn_norm = t(f"{p}.ffn_norm.weight")
+            ffn_norm = norm(f"{p}.ffn_norm.weight")
             w13 = decoder_ops.DecodeLinear(None, rows, gate_up=(t(f"{p}.feed_forward.w1.weight"),
                                                                 t(f"{p}.feed_forward.w3.weight")), in_scale=ffn_norm)
             if w13.in_scale_folded:
                 ffn_norm = torch.ones_like(ffn_norm)
-            self.layers.append(dict(attn=attn, attn_norm=t(f"{p}.attention_norm.weight"), ffn_norm=ffn_norm, w13=w13,
+            self.layers.append(dict(attn=attn, attn_norm=norm(f"{p}.attention_norm.weight"), ffn_norm=ffn_norm, w13=w13,
                                     w2=decoder_ops.DecodeLinear(t(f"{p}.feed_forward.w2.weight"), rows)))
         # tiled activations between the decode step's kernels where every projection that reads them is tiled
         self._tiled_acts = self.output.tiled and all(
