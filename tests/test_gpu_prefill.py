@@ -214,6 +214,28 @@ def test_layer_prefill_takes_unaligned_prompts(gpu):
     assert torch.equal(att.forward(x, mode="prefill"), att.forward(x.clone(), mode="prefill"))
 
 
+@pytest.mark.parametrize("kind", ["wider rows", "every other position", "fp32", "unaligned"])
+def test_layer_prefill_fills_caches_of_the_callers(gpu, kind):
+    """Row-major caches that a caller put into layer_past as views or in another type are filled as torch fills them."""
+    att, g = _layer(64, 32, 1, "rows", 1, 64)
+    x = torch.randn(1, 20, 256, generator=g).to(torch.bfloat16).cuda()
+    out = att._prefill_one(x[0], 1)
+    exp = [c.clone() for c in att.layer_past]
+
+    def other(c):
+        B, G, S, w = c.shape
+        if kind == "wider rows":
+            return torch.zeros(B, G, S, w + 16, dtype=c.dtype, device=c.device)[..., :w]
+        if kind == "every other position":
+            return torch.zeros(B, G, 2 * S, w, dtype=c.dtype, device=c.device)[:, :, ::2]
+        if kind == "fp32":
+            return torch.zeros_like(c, dtype=torch.float32)
+        return torch.zeros(1 + c.numel(), dtype=c.dtype, device=c.device)[1:].view(c.shape)
+    att.layer_past = [other(c) for c in att.layer_past]
+    assert torch.equal(att.forward(x, mode="prefill", user_id=1)[0], out)
+    assert all(torch.equal(c.to(torch.bfloat16), e) for c, e in zip(att.layer_past, exp))
+
+
 def test_layer_prefill_keeps_autograd(gpu):
     att, g = _layer(64, 64, 1, "rows", 1, 64)
     x = torch.randn(1, 20, 256, generator=g).cuda().requires_grad_()

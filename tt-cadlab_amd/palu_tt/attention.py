@@ -296,8 +296,9 @@ class PaluAttention(torch.nn.Module):
         x3 = x.reshape(-1, shape[-2], self.hidden_size).to(torch.bfloat16)          # [U, S, dim]
         U, S = x3.shape[0], x3.shape[1]
         assert 0 < S <= self.max_seq_len and user_id + U <= self.max_batch_size
-        if (U > 0 and user_id >= 0 and self.head_dim == 128 and decoder_ops.kernels_can_take(
-                x, self.wqkv.weight, self.wo, self.u_k, self.u_v, *(self._store(c) for c in self.layer_past))):
+        if (U > 0 and user_id >= 0 and self.head_dim == 128 and all(map(self._plain_cache, self.layer_past)) and
+                decoder_ops.kernels_can_take(x, self.wqkv.weight, self.wo, self.u_k, self.u_v,
+                                             *(self._store(c) for c in self.layer_past))):
             x2 = decoder_ops.aligned(x3.reshape(U * S, -1))
             return self._prefill_kernels(x2, U, user_id).reshape(*shape[:-1], self.hidden_size)
         outs = []
@@ -308,6 +309,12 @@ class PaluAttention(torch.nn.Module):
     @staticmethod
     def _store(cache):
         return cache if isinstance(cache, torch.Tensor) else cache.data
+
+    def _plain_cache(self, cache):
+        """Whether the fill kernel can write this cache (a caller may put its own tensors into layer_past: views and other
+        types are filled by torch)."""
+        t = self._store(cache)
+        return t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == self.wo.device and t.data_ptr() % 16 == 0
 
     def _prefill_kernels(self, x2, U, user):
         """The prompts of cache rows user .. user + U - 1 at once (x2 [U * S, dim]): one QKV projection, the latents (or
