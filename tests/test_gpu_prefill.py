@@ -4,6 +4,7 @@ The attention is compared with 64-bit torch on the same bf16 rows and fp32 table
 precision and rounds its result to bf16 once, so an output may be off by half a bf16 step at its value plus the
 fp32 computation's own error, which for these sizes stays below 4e-6 of the largest value of its row (fp32 attention
 through torch measures 2e-5 of the rms at worst over 2048 positions)."""
+import numpy as np
 import pytest
 import torch
 
@@ -212,6 +213,18 @@ def test_layer_prefill_takes_unaligned_prompts(gpu):
     x = buf[1:].view(1, 20, 256)
     assert x.data_ptr() % 16
     assert torch.equal(att.forward(x, mode="prefill"), att.forward(x.clone(), mode="prefill"))
+
+
+@pytest.mark.parametrize("as_type", [np.int64, torch.tensor])
+def test_layer_prefill_takes_integer_types_as_user_id(gpu, as_type):
+    att, g = _layer(64, 64, 1, "tiled", 1, 64)
+    x = torch.randn(1, 20, 256, generator=g).to(torch.bfloat16).cuda()
+    out = att.forward(x, mode="prefill", user_id=1)
+    exp = [c.data.clone() for c in att.layer_past]
+    for c in att.layer_past:
+        c.data.zero_()
+    assert torch.equal(att.forward(x, mode="prefill", user_id=as_type(1)), out)
+    assert all(torch.equal(c.data, e) for c, e in zip(att.layer_past, exp))
 
 
 @pytest.mark.parametrize("kind", ["wider rows", "every other position", "fp32", "unaligned"])

@@ -300,7 +300,7 @@ class PaluAttention(torch.nn.Module):
                 decoder_ops.kernels_can_take(x, self.wqkv.weight, self.wo, self.u_k, self.u_v,
                                              *(self._store(c) for c in self.layer_past))):
             x2 = decoder_ops.aligned(x3.reshape(U * S, -1))
-            return self._prefill_kernels(x2, U, user_id).reshape(*shape[:-1], self.hidden_size)
+            return self._prefill_kernels(x2, U, int(user_id)).reshape(*shape[:-1], self.hidden_size)
         outs = []
         for u in range(U):
             outs.append(self._prefill_one(x3[u], user_id + u))
