@@ -115,6 +115,20 @@ def test_decoder_above_64_rows_matches_lowrank_llama(gpu):
         _check(out, exp[:, S + t], f"decode step {t}")
 
 
+@pytest.mark.parametrize("ffn,shape", [(100, (2, 20)), (512, (1, 2, 20))])
+def test_prefill_of_shapes_past_the_kernels(gpu, ffn, shape, monkeypatch):
+    """An FFN width that is no multiple of 8 and prompts with one more dimension go the way of torch's operations."""
+    args = pm.ModelArgs(dim=256, n_layers=1, n_heads=4, n_kv_heads=2, vocab_size=320, ffn_dim=ffn, max_seq_len=64,
+                        max_batch_size=2)
+    net = pm.Transformer(args, pm.random_palu_state_dict(args, [64], [32], gpu, seed=5, std=0.05), gpu)
+    ids = (torch.arange(40, device=gpu) * 7).view(shape)
+    out = net.prefill(ids)
+    monkeypatch.setattr(pm.decoder_ops, "kernels_can_take", lambda *a: False)
+    exp = net.prefill(ids)
+    # the layer's own kernels against its torch path: bf16 roundings
+    assert out.shape == exp.shape and ((out - exp).norm() / exp.norm()).item() < 2.0 ** -6
+
+
 def _as_views(sd, keys):
     """The named tensors as views with the same values: off a 16-byte boundary, or (vectors) with a stride of 2."""
     for k in keys:

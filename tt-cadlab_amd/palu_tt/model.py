@@ -116,7 +116,9 @@ class Transformer(torch.nn.Module):
         logits of the last position of every row, [U, vocab]."""
         eps = self.args.norm_eps
         h = self.tok_embeddings[tokens]                                  # [U, S, dim]
-        if tokens.numel() > 0 and self.args.dim % 8 == 0 and self.args.dim <= 8192 and decoder_ops.kernels_can_take(h):
+        # what the RMSNorm and SwiGLU kernels take: rows of 8 up to 8192, [U, S] prompts, a gate / up pair of whole 8s
+        if (tokens.dim() == 2 and tokens.numel() > 0 and self.args.dim % 8 == 0 and self.args.dim <= 8192 and
+                all(L["w13"].n % 16 == 0 for L in self.layers) and decoder_ops.kernels_can_take(h)):
             return self._prefill_kernels(h, user_id)
         for L in self.layers:
             h = h + L["attn"].forward_prefill(rms_norm(h, L["attn_norm"], eps), user_id=user_id)
