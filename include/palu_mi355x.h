@@ -69,8 +69,8 @@ int palu_abi_version(void);
 
 /* Bytes of workspace palu_sdpa_decode / palu_flash_decode need for these shapes (0 when the
  * sequence is not split across workgroups). head_dim_v is the output width of the call. It holds the
- * split items' fp32 partials and one 8-byte chunk counter per (row, KV head); the launch merges the
- * partials itself and needs no particular contents on entry (counters of other calls count as zero).
+ * split items' fp32 partials and one 8-byte done flag per workgroup; the launch merges the
+ * partials itself and needs no particular contents on entry (a flag of another call does not count as set).
  * Calls that share a workspace must be ordered on one stream. */
 size_t palu_decode_workspace_bytes(int batch, int n_kv, int seq_len, int head_dim_v);
 

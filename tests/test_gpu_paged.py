@@ -6,11 +6,13 @@ contiguous rows through a random permutation of pages, rows have ragged lengths 
 middle of a page and of a 32-position block), and the mixed-rank shapes (r_k, r_v) = (32, 128) and
 (128, 64) with 64-token pages and lengths up to 32768 cover the paged configuration of the hot path.
 """
+import ctypes
+
 import pytest
 import torch
 
 from oracle import palu_oracle as ref
-from palu_tt import fused
+from palu_tt import _build, _native, fused
 from palu_tt.cache import LatentCache
 
 pytestmark = pytest.mark.gpu
@@ -196,13 +198,15 @@ def test_paged_stock_decode_matches_full_kv_oracle(gpu, layout):
     _check(out.cpu(), exp)
 
 
-def test_split_items_repeat_exactly_on_one_shared_workspace(gpu):
-    """Split items (8 rows x 8 KV heads on a 256-workgroup plan) merge inside the decode launch: each
-    chunk counts itself into an 8-byte counter of its item in the workspace, and the chunk that completes
-    the count merges the item. Two inputs alternate on one workspace that first holds stale counter words
-    (the fixed tag with a call number no launch carries and a nonzero count), with a call of other widths in between
-    whose partial slots overlay these calls' counters: every output must equal its input's first output
-    bit for bit, and match the oracle."""
+@pytest.mark.parametrize("refill", [False, True])
+def test_split_items_repeat_exactly_on_one_shared_workspace(gpu, refill):
+    """Split items (8 rows x 8 KV heads on a 256-workgroup plan) merge inside the decode launch: each chunk sets its
+    8-byte done flag in the workspace to the call's word (a fixed tag, the call number, 16 zero bits), and a chunk that
+    finds its whole item's flags set merges the item. Two inputs alternate on one workspace that first holds words of a
+    call number no launch carries (so that a flag compared without its call number counts as set at once), with a call of
+    other widths in between whose partial slots overlay these calls' flags; with refill, every call meets the words of
+    another call number instead, the neighbours of its own and those that differ in one bit among them. Every output must
+    equal its input's first output bit for bit, and match the oracle."""
     S, ps = 8192, 64
     cases = []
     for seed, r_k, r_v in ((1, 64, 64), (2, 64, 64), (3, 32, 128)):
@@ -210,16 +214,25 @@ def test_split_items_repeat_exactly_on_one_shared_workspace(gpu):
         lengths = torch.randint(1, S + 1, (8,), generator=g).tolist()
         lengths[0] = S
         cases.append(_case(8, S, r_k, r_v, ps, seed=seed, lengths=lengths))
-    from palu_tt import _native
     need = max(_native.load().palu_decode_workspace_bytes(8, 8, S, c[2].shape[-1]) for c in cases)
     assert need > 0, "the plan must split items for this test"
+    next_word = ctypes.CDLL(str(_build.library_path()))._ZN4palu10next_epochEv     # palu::next_epoch
+    next_word.restype, next_word.argtypes = ctypes.c_ulonglong, []
+    assert next_word() >> 48 == 0xA5C3
     ws = torch.empty(need // 8 + 1, dtype=torch.int64, device=gpu)
-    stale = (0xA5C3 << 48) | (0 << 16) | 5                 # call number 0 (no launch's), five chunks counted
-    ws.fill_(stale - (1 << 64))
+
+    def fill(number, low=0):
+        ws.fill_(((0xA5C3 << 48) | ((number & 0xFFFFFFFF) << 16) | low) - (1 << 64))
+    fill(0)
+    stale = [lambda n: (0,), lambda n: (n - 1,), lambda n: (n + 1,), lambda n: (n ^ 1,), lambda n: (n ^ 1 << 7,),
+             lambda n: (n ^ 1 << 15,), lambda n: (n ^ 1 << 16,), lambda n: (n ^ 1 << 31,), lambda n: (~n,),
+             lambda n: (n, 1), lambda n: (n, 1 << 15)]
     cos, sin = ref.cos_sin_tables(HD, S, THETA, LLAMA3)
     first = {}
     for it, i in enumerate([0, 1, 0, 2, 1, 0, 2, 1, 1, 0, 0]):
         q, k, v, u_k, pos, kp, vp, pt = cases[i]
+        if refill:
+            fill(*stale[it](((next_word() >> 16) & 0xFFFFFFFF) + 1))     # the next launch's number, changed
         out = _decode(gpu, q, kp, vp, u_k, pos, pt, S, "tiled", workspace=ws)
         if i not in first:
             first[i] = out
