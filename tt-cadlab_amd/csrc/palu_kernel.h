@@ -389,10 +389,6 @@ __device__ __forceinline__ int load_uniform(const int32_t* p, long long i) {
   return reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p))[i];
 }
 
-__device__ __forceinline__ float load_uniform_f(const float* p, long long i) {
-  return reinterpret_cast<const __attribute__((address_space(4))) float*>(reinterpret_cast<uintptr_t>(p))[i];
-}
-
 __device__ __forceinline__ int clamp_len(const DecodeArgs& a, int pos) {
   const int len = pos + 1;
   return len < 0 ? 0 : (len > a.S ? a.S : len);

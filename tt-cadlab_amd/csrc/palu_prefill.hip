@@ -21,7 +21,7 @@
 // probabilities multiply the bf16 latent rows (three MFMAs over r_v columns instead of six over 128) and u_v
 // is applied once per query at the end.
 //
-// Per query head and (query, key) pair 3 x 128 + 3 x r_v multiply-adds.
+// Per query head and (query, key) pair 3 x 128 + 3 x r_v multiply-adds, 3 x 128 + 6 x 128 where V is rebuilt.
 #include "palu_kernel.h"
 
 #include <algorithm>

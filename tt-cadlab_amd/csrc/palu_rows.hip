@@ -45,6 +45,8 @@ typedef __attribute__((address_space(1))) const void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
 constexpr int XS = 4;                     // activation stages in LDS
+constexpr int ROWS_MT = 8;                // 16-row activation tiles of a workgroup
+constexpr int ROWS_PER_CU = 2;            // workgroups that share a CU
 
 template <int MT, int RPW, bool SWIGLU>
 __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
@@ -251,7 +253,7 @@ int launch_rows(const RowsArgs& a0, hipStream_t s) {
 }
 
 struct RowsPlan {
-  int mt, rpw, ks;
+  int rpw, ks;
 };
 
 // Columns per workgroup (64 RPW) and k slices: the pair whose busiest CU finishes first, from a model in clocks. Per k
@@ -261,23 +263,20 @@ struct RowsPlan {
 // trip and a launch: 100 x 4096 x 14336 takes 139 us whole, 33.7 in 8 slices, 41.8 in 16; 2048 rows 226 whole, 234 in 2.
 // The model's pick was the fastest or within 4 % of it at 15 of 17 measured shapes (12 % off at the worst).
 RowsPlan rows_plan(int m, int n16, int kt_total, bool swiglu) {
-  static const int cfg[2][2] = {{8, 4}, {8, 2}};
-  RowsPlan best{8, 4, 1};
+  RowsPlan best{4, 1};
   double cost = 1e300;
-  for (const auto& c : cfg) {
-    const int mt = c[0], rpw = c[1];
-    const long long mblk = (m + 16 * mt - 1) / (16 * mt), ncol = (n16 + 4 * rpw - 1) / (4 * rpw);
-    const int per_cu = mt * rpw <= 32 ? 2 : 1;            // workgroups that share a CU
+  for (const int rpw : {4, 2}) {
+    const long long mblk = (m + 16 * ROWS_MT - 1) / (16 * ROWS_MT), ncol = (n16 + 4 * rpw - 1) / (4 * rpw);
     for (int ks = 1; ks <= (swiglu ? 1 : 16); ks *= 2) {
       const int ktps = (kt_total + ks - 1) / ks;
       if (ks > 1 && ktps < 16) break;
-      const long long units = mblk * ncol * ks, slots = 256LL * per_cu;
-      const double mfma = 16.0 * mt * rpw, mem = (4.0 * rpw + mt) * 1024.0 / 40.0;
-      const double rounds = units <= slots ? (units <= 256 ? 1.0 : (double)per_cu) : (double)((units + slots - 1) / slots) * per_cu;
+      const long long units = mblk * ncol * ks, slots = 256LL * ROWS_PER_CU;
+      const double mfma = 16.0 * ROWS_MT * rpw, mem = (4.0 * rpw + ROWS_MT) * 1024.0 / 40.0;
+      const double rounds = units <= 256 ? 1.0 : (double)((units + slots - 1) / slots) * ROWS_PER_CU;
       const double t = rounds * (ktps * (mfma > mem ? mfma : mem) + 3000.0) + (ks > 1 ? 6000.0 + 2.0 * ks * m * n16 * 64 / 2000.0 : 0.0);
       if (t < cost * 0.999) {
         cost = t;
-        best = RowsPlan{mt, rpw, ks};
+        best = RowsPlan{rpw, ks};
       }
     }
   }
@@ -286,7 +285,7 @@ RowsPlan rows_plan(int m, int n16, int kt_total, bool swiglu) {
 
 template <bool SWIGLU>
 int dispatch_rows(const RowsPlan& p, const RowsArgs& a, hipStream_t s) {
-  return p.rpw == 4 ? launch_rows<8, 4, SWIGLU>(a, s) : launch_rows<8, 2, SWIGLU>(a, s);
+  return p.rpw == 4 ? launch_rows<ROWS_MT, 4, SWIGLU>(a, s) : launch_rows<ROWS_MT, 2, SWIGLU>(a, s);
 }
 
 bool rows_shape_ok(int m, int n, int k) { return m > 0 && n > 0 && n % 16 == 0 && k > 0 && k % 32 == 0; }

@@ -542,9 +542,10 @@ class DecodeLinear:
     up pair, gate_up=(w_gate, w_up) instead: y = silu(x @ w_gate.T) * (x @ w_up.T)). For up to 64 rows
     (and n % 16 == 0, k % 32 == 0) the weight is held only in the tiled order of linear_tiled, with the
     work split linear_plan suggests (or rtw / ks; single_slice: one k slice, for the fused residual and
-    QKV epilogues) and a workspace for its split partials; otherwise it stays as it is and the call is
-    torch's F.linear. plain() returns the weight in the nn.Linear layout ([gate; up] for a pair; a fresh
-    copy when tiled), for the prefill's many-row products. in_scale (a gate / up pair only): the weight of
+    QKV epilogues) and a workspace for the decode step's split partials; otherwise it stays as it is and the
+    call is torch's F.linear. rows() is the product of a prefill's rows over the weight as it is held. plain()
+    returns the weight in the nn.Linear layout ([gate; up] for a pair; a fresh copy when tiled), for the torch
+    path of the prefill (autograd, tracing, shapes the kernels don't take). in_scale (a gate / up pair only): the weight of
     the RMSNorm in front of the pair, folded into the tiled weight's columns (w * in_scale) so that
     norm_eps calls take the normalisation into the same launch (linear_swiglu_rmsnorm); in_scale_folded
     says whether it was (only a tiled pair folds it), and then plain() holds the folded weight too."""
