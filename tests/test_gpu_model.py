@@ -115,6 +115,37 @@ def test_decoder_above_64_rows_matches_lowrank_llama(gpu):
         _check(out, exp[:, S + t], f"decode step {t}")
 
 
+def test_short_prefills_and_decode_on_two_streams(gpu):
+    """Prompts of 20 and 60 positions prefilled on two streams at once, decode steps running on one of them: logits and
+    caches equal, bit for bit, those of the same calls one after the other (no scratch is shared between them)."""
+    args = pm.ModelArgs(dim=256, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=320, ffn_dim=8192, max_seq_len=64,
+                        max_batch_size=3)
+    net = pm.Transformer(args, pm.random_palu_state_dict(args, [64, 32], [32, 64], gpu, seed=6, std=0.05), gpu)
+    net.set_deterministic(True)
+    assert net.layers[0]["w2"].ks > 1, "the down projection must split for this test"
+    ids = [(torch.arange(n, device=gpu) * 11 + n).remainder(320)[None] for n in (20, 60)]
+    tok, pos = torch.tensor([3, 5, 7], device=gpu), torch.full((3,), 63, dtype=torch.int32, device=gpu)
+    caches = lambda: [c.data.clone() for L in net.layers for c in L["attn"].layer_past]
+    alone = [net.prefill(t, user_id=u) for u, t in enumerate(ids)]
+    step = net.decode(tok, pos)
+    held = caches()
+    streams = [torch.cuda.Stream() for _ in ids]
+    torch.cuda.synchronize()
+    for _ in range(15):
+        outs, steps = [], []
+        for u, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs.append(net.prefill(ids[u], user_id=u))
+        torch.cuda.synchronize()               # the step reads the caches that the prefills write
+        with torch.cuda.stream(streams[0]):
+            steps.append(net.decode(tok, pos))
+        with torch.cuda.stream(streams[1]):
+            outs.append(net.layers[1]["w2"].rows(net.layers[1]["w13"].rows(net.tok_embeddings[ids[1][0]])))
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], alone[0]) and torch.equal(outs[1], alone[1]) and torch.equal(steps[0], step)
+        assert all(torch.equal(a, b) for a, b in zip(caches(), held))
+
+
 @pytest.mark.parametrize("ffn,shape", [(100, (2, 20)), (512, (1, 2, 20))])
 def test_prefill_of_shapes_past_the_kernels(gpu, ffn, shape, monkeypatch):
     """An FFN width that is no multiple of 8 and prompts with one more dimension go the way of torch's operations."""
