@@ -1,6 +1,6 @@
 // Prefill attention of one layer over whole prompts: causal attention of every prompt position over the
-// prompt's own latents, with the precision of an fp32 attention (fp32 K, V, scores, probabilities and sums),
-// as PaluAttention's prefill has always computed it (reference palu_tt/attention.py:380-480). Replaces the
+// prompt's own latents, as near to exact as an fp32 attention (fp32 K, V, probabilities and sums, score operands
+// of 22 bits; below), which PaluAttention's prefill computed before (reference palu_tt/attention.py:380-480). Replaces the
 // chain of torch ops (casts, einsum rebuilds, RoPE, head repeats, fp32 SDPA) with three launches over the QKV
 // projection's bf16 output rows:
 //   1. palu_latent_fill: the new latents (or, on the stock K path, the rotated keys) into the caches;
@@ -333,9 +333,9 @@ __global__ __launch_bounds__(256) void palu_prefill_rebuild_kernel(const Prefill
 // and written at its end, so that the first K tiles of j + 1 can be read before the barrier) and every K tile read from LDS
 // feeds up to 2 NG MFMAs. K tiles are read one dim block ahead of their products and V tiles ahead of the softmax (two
 // buffers and reads where the compiler put them: 4096 positions at r 64 / 64 312 -> 309 us with the rebuild, 2048 at 64 /
-// 128 183 -> 172). Running half of the waves half a record behind the others, so that one half's softmax meets the other's
-// products, was slower (323 us). At 4096 positions the matrix cores are busy 44 % and the vector ALU 35 % of the time: a
-// softmax of eight keys costs a lane about 100 instructions beside 36 MFMAs. Scores are computed transposed
+// 128 183 -> 172, one box; 320 to 325 and 170 on others, with a scale to every key). Running half of the waves half a record behind the others, so that one half's softmax meets the other's
+// products, was slower (323 us). At 4096 positions the matrix cores are busy 46 % and the vector ALU 38 % of the time: a
+// softmax of eight keys costs a lane about 110 instructions beside 36 MFMAs. Scores are computed transposed
 // (keys x rows), so a lane holds eight keys of one row per column group: softmax in the exp2 domain with a lazily
 // refreshed maximum (cross-lane work only when a score passes it by 2^8), probabilities split into planes in
 // place, and they are the PV product's operand as they stand.

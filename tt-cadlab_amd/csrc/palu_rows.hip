@@ -12,11 +12,13 @@
 // LDS feeds RPW MFMAs and a weight tile MT. Two workgroups share a CU.
 //
 // Bound: MFMA from some 500 rows on, the weight stream below. Measured (MI355X, weights rotated past the caches; the
-// library GEMM on an nn.Linear-layout copy, without the time to make the copy, in brackets): 2048 x 28672 x 4096
-// with SwiGLU 427 us = 1.13 PFLOP/s (391), 2048 x 4096 x 14336 220 us (222), 512 x 28672 x 4096 134 (104), 128 x 28672 x
-// 4096 59.5 (57.1), 300 x 4096 x 14336 66 (74), 100 x 4096 x 14336 33.5 (49.4). First forms: activations through registers
-// (one stage ahead) 535 us at the first shape; 256-row workgroups with one wave per SIMD 653 to 740 us (the 256
-// accumulators and the stages do not fit without copies); waits left to the compiler 543 us.
+// library GEMM on an nn.Linear-layout copy, without the time to make the copy and without SwiGLU, in brackets; two boxes
+// where they differ): 2048 x 28672 x 4096 with SwiGLU 428 us = 1.13 PFLOP/s (355 to 391), 2048 x 4096 x 14336 220 (208
+// to 222), 4096 x 5120 x 4096 182 (145), 1554 x 5376 x 4096 107 (72), 512 x 28672 x 4096 129 (100), 128 x 28672 x 4096
+// 56 (56), 300 x 4096 x 14336 62 (74), 100 x 4096 x 14336 34 (51). So the library's product is the faster one at full
+// shapes; the copy it needs takes longer than the difference. First forms: activations through registers (one stage
+// ahead) 535 us at the first shape; 256-row workgroups with one wave per SIMD 653 to 740 us (the 256 accumulators and
+// the stages do not fit without copies); waits left to the compiler 543 us.
 //
 // Work order: the workgroups that share a weight column block run next to each other on one XCD (ids 8 apart), so the
 // weight comes from memory once and from that XCD's L2 for the other row blocks.
