@@ -157,9 +157,10 @@ __global__ __launch_bounds__(256, 2) void palu_rows_kernel(const RowsArgs a) {
     }
     load_x(xs0, 0);
     load_x(xs1, 1);
+    __builtin_amdgcn_sched_barrier(0);                    // stage 2's copies last: the wait below is for all but them
     load_x(xs2, 2);
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | XPW);             // all but stage 2: the loop counts on loads in steady order
+    __builtin_amdgcn_s_waitcnt(0x0F70 | XPW);             // the loop counts on loads in steady order
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     int s = 0;
