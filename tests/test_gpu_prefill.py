@@ -1,8 +1,8 @@
 """The prefill attention and cache-fill kernels (palu_prefill_attention, palu_latent_fill).
 
-The attention is compared with 64-bit torch on the same bf16 rows and fp32 tables. The kernel computes in fp32
-precision and rounds its result to bf16 once, so an output may be off by half a bf16 step at its value plus the
-fp32 computation's own error, which for these sizes stays below 4e-6 of the largest value of its row (fp32 attention
+The attention is compared with 64-bit torch on the same bf16 rows and fp32 tables. The kernel keeps fp32 sums, takes
+score operands with 22 bits and rounds its result to bf16 once, so an output may be off by half a bf16 step at its value
+plus the computation's own error, which for these sizes stays below 4e-6 of the largest value of its row (fp32 attention
 through torch measures 2e-5 of the rms at worst over 2048 positions)."""
 import numpy as np
 import pytest
