@@ -160,6 +160,20 @@ def test_prefill_of_shapes_past_the_kernels(gpu, ffn, shape, monkeypatch):
     assert out.shape == exp.shape and ((out - exp).norm() / exp.norm()).item() < 2.0 ** -6
 
 
+def test_prefill_keeps_forward_mode_tangents_of_weights(gpu):
+    """A dual norm weight: the prefill's logits carry its tangent (d logits = logits with the tangent as the weight)."""
+    args = pm.ModelArgs(dim=256, n_layers=1, n_heads=4, n_kv_heads=2, vocab_size=320, ffn_dim=512, max_seq_len=64,
+                        max_batch_size=2)
+    net = pm.Transformer(args, pm.random_palu_state_dict(args, [64], [32], gpu, seed=5, std=0.05), gpu)
+    ids, w = torch.arange(40, device=gpu).view(2, 20) * 7, net.norm_w
+    net.norm_w = 2 * w
+    twice = net.prefill(ids)
+    with torch.autograd.forward_ad.dual_level():
+        net.norm_w = torch.autograd.forward_ad.make_dual(w, 2 * w)
+        tangent = torch.autograd.forward_ad.unpack_dual(net.prefill(ids)).tangent
+    assert tangent is not None and ((tangent - twice).norm() / twice.norm()).item() < 2.0 ** -6   # bf16 roundings
+
+
 def _as_views(sd, keys):
     """The named tensors as views with the same values: off a 16-byte boundary, or (vectors) with a stride of 2."""
     for k in keys:

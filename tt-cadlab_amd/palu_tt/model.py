@@ -118,7 +118,9 @@ class Transformer(torch.nn.Module):
         h = self.tok_embeddings[tokens]                                  # [U, S, dim]
         # what the RMSNorm and SwiGLU kernels take: rows of 8 up to 8192, [U, S] prompts, a gate / up pair of whole 8s
         if (tokens.dim() == 2 and tokens.numel() > 0 and self.args.dim % 8 == 0 and self.args.dim <= 8192 and
-                all(L["w13"].n % 16 == 0 for L in self.layers) and decoder_ops.kernels_can_take(h)):
+                all(L["w13"].n % 16 == 0 for L in self.layers) and decoder_ops.kernels_can_take(
+                    h, self.norm_w, self.output.weight, *(t for L in self.layers for t in (
+                        L["attn_norm"], L["ffn_norm"], L["w13"].weight, L["w2"].weight)))):
             return self._prefill_kernels(h, user_id)
         for L in self.layers:
             h = h + L["attn"].forward_prefill(rms_norm(h, L["attn_norm"], eps), user_id=user_id)
